@@ -1,0 +1,91 @@
+// INT4 group-32 instances of the wide GEMM tile, and the choice of tile and split for both formats.
+#include "gemm_wide_kernel.h"
+
+#include <algorithm>
+
+namespace moss {
+namespace {
+
+// Nanoseconds a workgroup takes per K step of 64, by tile (columns JT = 1 .. 5): `alone`, with a CU to
+// itself, and `shared`, per workgroup with two on the CU.  Medians over M = 5 .. 2048 on the four
+// projections of the 4096 / 12288 model (K 4096 and 12288, N 4096 .. 24576), within 10% of nearly all
+// of them; 0: no such instance (R = 2 below 3 token tiles lost to R = 1 everywhere, and INT4 at 2 x 5
+// spills).
+struct StepCost {
+    int alone[5], shared[5];
+};
+constexpr StepCost kStepCost[2][2] = {
+    {{{345, 390, 430, 540, 620}, {262, 345, 400, 530, 580}}, {{0, 0, 760, 1000, 0}, {0, 0, 720, 940, 0}}},
+    {{{330, 370, 400, 470, 560}, {275, 320, 385, 520, 555}}, {{0, 0, 740, 900, 1056}, {0, 0, 680, 880, 1100}}},
+};
+
+template <int R, int JT>
+int launch_tile(WideEpilogue epi, const WidePlan& p, const WideArgs& a, hipStream_t st) {
+    const int bn = (epi == kWideSilu ? 64 : 128) * R;
+    const dim3 grid((unsigned)(((a.M + 32 * JT - 1) / (32 * JT)) * ((a.N + bn - 1) / bn) * p.split));
+#define MOSS_WIDE(EPI)                                                                                               \
+    hipLaunchKernelGGL((gemm_wide_kernel<kInt4G32, R, JT, EPI>), grid, dim3(256), 0, st, (const uint16_t*)a.x,        \
+                       (const uint8_t*)a.qw, (const uint16_t*)a.sc, (const uint8_t*)a.zp, a.row_scale, (uint16_t*)a.y, \
+                       a.part, a.M, a.N, a.K, p.split, a.qr)
+    if (epi == kWideSplit) MOSS_WIDE(kWideSplit);
+    else if (epi == kWideSilu) MOSS_WIDE(kWideSilu);
+    else if (epi == kWideQkRope) MOSS_WIDE(kWideQkRope);
+    else MOSS_WIDE(kWidePlain);
+#undef MOSS_WIDE
+    return moss_launch_status();
+}
+
+}  // namespace
+
+// Whole blocks of four K steps and 4-output stores; INT4: the 8 zero bytes of every block on one
+// nibble side of their 128-group chunk (the last chunk a multiple of 16 groups long).  The weight lies
+// within the 32-bit offsets of the buffer instructions.
+bool wide_shape(int fmt, int K, int nw) {
+    if (nw % 4 || K % (4 * kStep) || (long long)nw * K / (fmt == kInt4G32 ? 2 : 1) >= 1ll << 31) return false;
+    const int G = K / 32;
+    return fmt == kFp8E4M3 || (G % 16 == 0 && (G % 128) % 16 == 0);
+}
+
+// The expected time of each tile and split is what the step costs above give for the workgroups per CU,
+// not less than the weights' bytes at 4.5 TB/s, and for a split the partial sums written and read back
+// (8 bytes each at 5 TB/s) and the launch that adds them.  A split leaves every workgroup at least two
+// blocks of K and its partials fit 32 MiB.
+WidePlan wide_plan(int fmt, int M, int K, int nw, int max_split) {
+    WidePlan best{1, 1, 1};
+    double least = 1e30;
+    const double wbytes = (double)nw * K * (fmt == kInt4G32 ? 0.5625 : 1.0);
+    for (int r = 1; r <= 2; ++r)
+        for (int jt = 1; jt <= 5; ++jt) {
+            const StepCost& c = kStepCost[fmt][r - 1];
+            if (!c.alone[jt - 1] || (jt > 1 && 32 * (jt - 1) >= M)) continue;
+            const long tiles = (long)((M + 32 * jt - 1) / (32 * jt)) * ((nw + 128 * r - 1) / (128 * r));
+            for (int split = 1; split <= max_split; split *= 2) {
+                const int steps = K / kStep / split;
+                if (split > 1 && (K / kStep % (4 * split) || steps < 8 || (long long)split * M * nw * 4 > 32ll << 20)) break;
+                const long per_cu = (tiles * split + 255) / 256;
+                const double ns = per_cu == 1 ? c.alone[jt - 1] : (double)per_cu * c.shared[jt - 1];
+                double us = 3.5 + std::max(steps * ns / 1000, wbytes / 4.5e6);
+                if (split > 1) us += 2.5 + (double)split * M * nw * 8 / 5e6;
+                if (us < least) {
+                    least = us;
+                    best = {r, jt, split};
+                }
+            }
+        }
+    return best;
+}
+
+int wide_launch_w4(WideEpilogue epi, const WidePlan& p, const WideArgs& a, hipStream_t st) {
+    switch (10 * p.r + p.jt) {
+        case 11: return launch_tile<1, 1>(epi, p, a, st);
+        case 12: return launch_tile<1, 2>(epi, p, a, st);
+        case 13: return launch_tile<1, 3>(epi, p, a, st);
+        case 14: return launch_tile<1, 4>(epi, p, a, st);
+        case 15: return launch_tile<1, 5>(epi, p, a, st);
+        case 23: return launch_tile<2, 3>(epi, p, a, st);
+        case 24: return launch_tile<2, 4>(epi, p, a, st);
+    }
+    return (int)hipErrorInvalidValue;
+}
+
+}  // namespace moss

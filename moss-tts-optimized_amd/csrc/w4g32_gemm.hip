@@ -11,11 +11,10 @@
 // epilogue (src/moss_tts/_runtime/fused_mlp.py:20-21).  The fp8 MFMA forms are not used:
 // they would round the bf16 activations to e4m3 as well.
 //
-// INT4 takes the register-weight tile wherever its shape conditions hold (reg_tile_shape): the
-// dequantized weights are the MFMA's A operand straight from the registers that dequantize them,
-// and only the activations are staged in LDS (w4g32_gemm_t_kernel up to 64 tokens per tile;
-// w4g32_gemm_tdma_kernel, whose activations go from global memory to LDS without registers, for
-// 128).  FP8, other INT4 shapes and misaligned scale or zero-point pointers take the LDS tiles:
+// Both formats take the wide tile (gemm_wide_kernel.h) wherever its shape conditions hold
+// (wide_shape) and the few-token paths below do not win (choose_wide).  w4g32_gemm_tdma_kernel, the
+// 128-token tile with 64-bit addresses, takes INT4 weights past 32-bit offsets; other shapes and
+// misaligned scale or zero-point pointers take the LDS tiles:
 //
 // LDS tiles: BM x BN outputs (BM, BN in {64, 128}) per 256-thread workgroup, 2 x 2 waves of
 // (BM/2) x (BN/2), K in steps of 64 (two quantization groups).  Pipeline: two LDS buffers and
@@ -28,7 +27,7 @@
 // Tile order: logical tiles are n-major with the M tiles of one N tile adjacent, and the
 // workgroup id is remapped so that consecutive logical tiles run on the same XCD (workgroups
 // are dealt to the 8 XCDs round-robin), so a weight tile is fetched into one L2.
-#include "common.h"
+#include "gemm_wide.h"
 
 #include <mutex>
 #include <type_traits>
@@ -48,8 +47,6 @@ constexpr int kXcds = 8;
 // accumulators leave room for two stages at two waves per SIMD.
 template <int BM, int BN>
 constexpr int stages_for() { return BM == 128 && BN == 128 ? 2 : 4; }
-
-enum WeightFormat { kInt4G32 = 0, kFp8E4M3 = 1 };
 
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 
@@ -305,20 +302,15 @@ __global__ __launch_bounds__(256) void w4g32_gemm_kernel(const uint16_t* __restr
 
 // Weight-stationary-in-registers INT4 tile (Y^T = W X^T): the dequantized weights are the MFMA's
 // A operand, formed in the registers of the lane that feeds them, so they never pass through
-// LDS; only the activation tile does.  A workgroup covers 128 weight rows and
-// BM = 32 JT tokens: wave w owns weight rows n0 + 32 w .. + 31 and every token (JT MFMA tiles
-// of 32 x 32).  In a K step of 64, lane l takes row n0 + 32 w + (l & 31) and the 32-wide half
-// (l >> 5) of the step: its 32 weights are the A operands of the step's 4 MFMAs (8 per MFMA),
-// and MFMA kk meets the activations x[m][32 (l >> 5) + 8 kk .. + 8] of the same lane, so both
-// operands walk K in the same order: one group of 32 codes (16 bytes) per lane and step,
-// dequantized bit-exactly.  (FP8 weights measured slower in this tile than in the LDS tiles at
-// M <= 128 and take those.)
-// Vector-memory requests are counted per 64-byte segment an instruction touches, so every load
-// is shaped to touch few: eight consecutive threads copy one token row's 128 bytes of a step, and
-// the scales and zero points of a row come once per block of kTs steps (8 groups: 16 bytes
-// of scales, 8 zero bytes that all hold the same nibble half when the row's last 128-group
-// chunk is a multiple of 16 groups long).  Weights travel kTs steps ahead (HBM), activations
-// two steps ahead (mostly L2 hits), scales and zeros one block ahead.
+// LDS; only the activation tile does.  A workgroup covers 128 weight rows and 128 tokens: wave w owns
+// weight rows n0 + 32 w .. + 31 and every token (4 MFMA tiles of 32 x 32).  In a K step of 64, lane l
+// takes row n0 + 32 w + (l & 31) and the 32-wide half (l >> 5) of the step: its 32 weights are the A
+// operands of the step's 4 MFMAs (8 per MFMA), and MFMA kk meets the activations
+// x[m][32 (l >> 5) + 8 kk .. + 8] of the same lane: one group of 32 codes (16 bytes) per lane and step,
+// dequantized bit-exactly.  The scales and zero points of a row come once per block of kTs steps (8
+// groups: 16 bytes of scales, 8 zero bytes that all hold the same nibble half when the row's last
+// 128-group chunk is a multiple of 16 groups long).  Weights travel kTs steps ahead, activations one
+// step, scales and zeros one block.
 constexpr int kTs = 4;
 
 struct TBlock {
@@ -327,147 +319,11 @@ struct TBlock {
     uint32_t zsh;
 };
 
-// SPLIT: gridDim.y workgroups share a tile, each summing a contiguous K range of whole blocks
-// into fp32 partials part[blockIdx.y, M, N], reduced by gemm_reduce.
-template <int JT, bool SPLIT>
-__global__ __launch_bounds__(256) void w4g32_gemm_t_kernel(const uint16_t* __restrict__ X, const uint4* __restrict__ qw,
-                                                           const uint16_t* __restrict__ sc,
-                                                           const uint8_t* __restrict__ zp, uint16_t* __restrict__ Y,
-                                                           float* __restrict__ part, int M, int N, int K) {
-    constexpr int BN = 128, BM = 32 * JT;
-    __shared__ __attribute__((aligned(16))) uint16_t Xs[2][BM][kLds];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int mt = (M + BM - 1) / BM, tiles = gridDim.x;
-    int tile = blockIdx.x;
-    if (tiles % kXcds == 0) tile = (blockIdx.x % kXcds) * (tiles / kXcds) + blockIdx.x / kXcds;
-    const int m0 = (tile % mt) * BM, n0 = (tile / mt) * BN;
-    const int G = K >> 5, steps = SPLIT ? K / kBK / gridDim.y : K / kBK;
-    const int kbase = SPLIT ? blockIdx.y * steps * kBK : 0;  // a multiple of kTs steps (8 groups)
-    // activation copy: thread t moves 16-byte chunk t % 8 of token rows t / 8 + 32 c, c < JT
-    // (rows clamped; those outputs are not stored)
-    const int xc = tid & 7, xr = tid >> 3;
-    const uint16_t* xrow[JT];
-#pragma unroll
-    for (int c = 0; c < JT; ++c) xrow[c] = X + (size_t)min(m0 + xr + 32 * c, M - 1) * K + kbase + 8 * xc;
-    // weights: this lane's row and 32-wide half of the step
-    const int half = lane >> 5;
-    const size_t wrow = (size_t)min(n0 + 32 * wave + (lane & 31), N - 1);
-
-    auto load_x = [&](u32x4_t (&x)[JT], int k0) {
-#pragma unroll
-        for (int c = 0; c < JT; ++c) x[c] = __builtin_bit_cast(u32x4_t, *reinterpret_cast<const uint4*>(xrow[c] + k0));
-    };
-    auto load_w = [&](uint4& w, int k0) { w = qw[wrow * G + ((kbase + k0) >> 5) + half]; };
-    auto load_blk = [&](TBlock& t, int blk) {
-        const int g = (kbase >> 5) + 8 * blk;
-        int zb;
-        zero_loc(g, G, zb, t.zsh);
-        t.s = *reinterpret_cast<const uint4*>(sc + wrow * G + g);
-        t.z = *reinterpret_cast<const uint2*>(zp + wrow * (G >> 1) + zb);
-    };
-    auto store_x = [&](const u32x4_t (&x)[JT], uint16_t (*xs)[kLds]) {
-#pragma unroll
-        for (int c = 0; c < JT; ++c) *reinterpret_cast<u32x4_t*>(&xs[xr + 32 * c][8 * xc]) = x[c];
-    };
-
-    f32x16_t acc[JT];
-#pragma unroll
-    for (int j = 0; j < JT; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[j][e] = 0.f;
-
-    const int blocks = steps / kTs;
-    uint4 cw[kTs];
-    u32x4_t xv[2][JT];
-    TBlock cur, nxt;
-    load_blk(cur, 0);
-    load_blk(nxt, min(1, blocks - 1));
-#pragma unroll
-    for (int i = 0; i < kTs; ++i) load_w(cw[i], min(i, steps - 1) * kBK);
-    load_x(xv[0], 0);
-    load_x(xv[1], min(1, steps - 1) * kBK);
-    pin();
-    store_x(xv[0], Xs[0]);
-    __syncthreads();
-    const MixedUnpack mu = make_mixed_unpack();
-    for (int blk = 0; blk < blocks; ++blk) {
-        const int st = blk * kTs;
-#pragma unroll
-        for (int i = 0; i < kTs; ++i) {
-            const int s = st + i;
-            // all activation operands of the step first: their LDS latency is hidden behind the
-            // dequantization below instead of being exposed before each MFMA
-            const uint16_t (*xs)[kLds] = Xs[i % 2];
-            bf16x8_t b[4][JT];
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk)
-#pragma unroll
-                for (int j = 0; j < JT; ++j)
-                    b[kk][j] = *reinterpret_cast<const bf16x8_t*>(&xs[32 * j + (lane & 31)][32 * half + 8 * kk]);
-            pin();
-            // this step's A operands (group 8 blk + 2 i + half of this lane's row), in registers
-            uint32_t wf[4][4];
-            {
-                const uint32_t sw = i == 0 ? cur.s.x : i == 1 ? cur.s.y : i == 2 ? cur.s.z : cur.s.w;
-                const uint32_t zw = i < 2 ? cur.z.x : cur.z.y;
-                const uint32_t zq = (zw >> (8 * (2 * (i & 1) + half) + cur.zsh)) & 15u;
-                const GroupDequant gd = group_dequant(sw >> (16 * half), zq);
-                const uint32_t words[4] = {cw[i].x, cw[i].y, cw[i].z, cw[i].w};
-#pragma unroll
-                for (int kk = 0; kk < 4; ++kk)
-                    dequant_word_mixed(words[kk], mu, gd.s_lo, gd.s_hi, gd.s, gd.bias_bf16, gd.bias_f16, wf[kk]);
-            }
-            pin();
-            // slot i of the code ring is free once dequantized: codes of step s + kTs into it
-            load_w(cw[i], min(s + kTs, steps - 1) * kBK);
-            if (i == kTs - 1) {
-                cur = nxt;
-                load_blk(nxt, min(blk + 2, blocks - 1));
-            }
-            // the next step's activations into the other buffer, which every wave finished reading
-            // before the previous barrier (after the last step this writes clamped data nobody reads);
-            // their register slot then takes step s + 2
-            store_x(xv[(i + 1) % 2], Xs[(i + 1) % 2]);
-            load_x(xv[i % 2], min(s + 2, steps - 1) * kBK);
-            pin();
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk) {
-                const bf16x8_t a = __builtin_bit_cast(bf16x8_t, u32x4_t{wf[kk][0], wf[kk][1], wf[kk][2], wf[kk][3]});
-#pragma unroll
-                for (int j = 0; j < JT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[kk][j], acc[j], 0, 0, 0);
-            }
-            __syncthreads();
-        }
-    }
-    // C[n][m] of the 32 x 32 tile (n0 + 32 wave, m0 + 32 j): lane l, element e -> n row
-    // 8 (e / 4) + 4 (l / 32) + e % 4, m column l % 32; the four e of a quad are consecutive n
-    // (N % 4 == 0: a quad is all in range or all out)
-#pragma unroll
-    for (int j = 0; j < JT; ++j) {
-        const int m = m0 + 32 * j + (lane & 31);
-        if (m >= M) continue;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int n = n0 + 32 * wave + 8 * q + 4 * (lane >> 5);
-            if (n >= N) continue;
-            const float v0 = acc[j][4 * q], v1 = acc[j][4 * q + 1], v2 = acc[j][4 * q + 2], v3 = acc[j][4 * q + 3];
-            if constexpr (SPLIT) {
-                *reinterpret_cast<float4*>(part + ((size_t)blockIdx.y * M + m) * N + n) = make_float4(v0, v1, v2, v3);
-            } else {
-                uint2 o;
-                o.x = pack_bf16x2(v0, v1);
-                o.y = pack_bf16x2(v2, v3);
-                *reinterpret_cast<uint2*>(Y + (size_t)m * N + n) = o;
-            }
-        }
-    }
-}
-
-// The 128-token register-weight tile (M > 64) with the activations copied from global memory
-// straight into LDS (global_load_lds_dwordx4: lane i of an instruction writes bytes 16 i .. + 15
-// of a 1 KiB span), so no registers stage them and no LDS stores are issued: 150-152 VGPRs, three
-// workgroups per CU (768 gate||up tiles at M = 512 run in one round instead of 1.5).  Weights,
-// operands, MFMA order and results are those of w4g32_gemm_t_kernel<4, SPLIT>, bit for bit.
+// The activations are copied from global memory straight into LDS (global_load_lds_dwordx4: lane i of
+// an instruction writes bytes 16 i .. + 15 of a 1 KiB span), so no registers stage them and no LDS
+// stores are issued: 150-152 VGPRs, three workgroups per CU.  Its addresses are 64-bit; within 32-bit
+// offsets the wide tile is the faster one (M = 2048, K = 4096, N = 24576: 357 against 503 us) and takes
+// the call.  MFMA order and results are those of the wide tile, bit for bit.
 // LDS layout: two buffers of 128 token rows x 128 bytes (one K step), chunk c (8 bf16) of row r
 // stored at position c ^ (r & 7) ^ ((r >> 3) & 1): the 16 lanes that read one chunk of 16
 // consecutive rows in one LDS cycle (64 banks) hit 16 different 16-byte bank groups (r & 7 alone
@@ -498,18 +354,6 @@ __device__ __forceinline__ void cbar() { asm volatile("" ::: "memory"); }
 // the K/V cache write as its epilogue (N = 48 heads of 128: 32 query, 8 key, 8 value heads, one
 // head per 128-wide tile); Y receives the query heads [M, 32, 128].  Equal bit for bit to the
 // unsplit GEMM followed by moss_qk_norm_rope_kv with cos/sin rows taken by position.
-struct QkRope {
-    const uint16_t* q_weight;  // [128] head RMSNorm weights
-    const uint16_t* k_weight;
-    const uint16_t* cos_t;  // [L, 128], row = position
-    const uint16_t* sin_t;
-    uint16_t* k_cache;  // [8, L, 128]
-    uint16_t* v_cache;
-    const int64_t* positions;  // [M], clamped into 0 .. L - 1
-    int L;
-    float eps;
-};
-
 template <bool SPLIT, bool SILU = false, bool QKR = false>
 __global__ __launch_bounds__(256, 3) void w4g32_gemm_tdma_kernel(const uint16_t* __restrict__ X, const uint4* qw,
                                                               const uint16_t* sc, const uint8_t* zp,
@@ -756,7 +600,8 @@ __global__ __launch_bounds__(256, 3) void w4g32_gemm_tdma_kernel(const uint16_t*
         }
         return;
     }
-    // C[n][m] of the 32 x 32 tile (n0 + 32 wave, m0 + 32 j): as in w4g32_gemm_t_kernel
+    // C[n][m] of the 32 x 32 tile (n0 + 32 wave, m0 + 32 j): lane l, element e -> n row 8 (e / 4) +
+    // 4 (l / 32) + e % 4, m column l % 32; the four e of a quad are consecutive n
 #pragma unroll
     for (int j = 0; j < JT; ++j) {
         const int m = m0 + 32 * j + (lane & 31);
@@ -778,25 +623,52 @@ __global__ __launch_bounds__(256, 3) void w4g32_gemm_tdma_kernel(const uint16_t*
     }
 }
 
+// The S partials of 4 outputs added in z order from 0, loaded 4 at a time before they are added.
+__device__ __forceinline__ float4 sum_parts(const float* __restrict__ part, size_t mn, int S) {
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int z0 = 0; z0 < S; z0 += 4) {
+        float4 v[4];
+#pragma unroll
+        for (int z = 0; z < 4; ++z)
+            if (z0 + z < S) v[z] = *reinterpret_cast<const float4*>(part + (z0 + z) * mn);
+#pragma unroll
+        for (int z = 0; z < 4; ++z)
+            if (z0 + z < S) {
+                acc.x += v[z].x;
+                acc.y += v[z].y;
+                acc.z += v[z].z;
+                acc.w += v[z].w;
+            }
+    }
+    return acc;
+}
+
 // y[m, n] = bf16(scale[n] * sum_z part[z, m, n]), z ascending; 4 outputs per thread (N % 4 == 0).
 __global__ __launch_bounds__(256) void gemm_reduce(const float* __restrict__ part, const float* __restrict__ row_scale,
                                                    uint16_t* __restrict__ Y, int MN, int N, int S) {
     const int i = 4 * (blockIdx.x * blockDim.x + threadIdx.x);
     if (i >= MN) return;
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int z = 0; z < S; ++z) {
-        const float4 v = *reinterpret_cast<const float4*>(part + (size_t)z * MN + i);
-        acc.x += v.x;
-        acc.y += v.y;
-        acc.z += v.z;
-        acc.w += v.w;
-    }
+    const float4 acc = sum_parts(part + i, (size_t)MN, S);
     const int n = i % N;  // the 4 outputs share a row
     float4 s = make_float4(1.f, 1.f, 1.f, 1.f);
     if (row_scale) s = make_float4(row_scale[n], row_scale[n + 1], row_scale[n + 2], row_scale[n + 3]);
     uint2 o;
     o.x = pack_bf16x2(acc.x * s.x, acc.y * s.y);
     o.y = pack_bf16x2(acc.z * s.z, acc.w * s.w);
+    *reinterpret_cast<uint2*>(Y + i) = o;
+}
+
+// The same over [M, 2 N] gate||up sums followed by the SiLU*mul: Y[m, n] = bf16(bf16(silu(g)) u) of the
+// bf16-rounded sums g = [m, n], u = [m, N + n], bit for bit what gemm_reduce and moss_silu_mul give.
+__global__ __launch_bounds__(256) void gemm_reduce_silu(const float* __restrict__ part, uint16_t* __restrict__ Y,
+                                                        int MN, int N, int S) {
+    const int i = 4 * (blockIdx.x * blockDim.x + threadIdx.x);  // output index in [M, N], N % 4 == 0
+    if (i >= MN) return;
+    const size_t at = (size_t)(i / N) * 2 * N + i % N, mn2 = 2 * (size_t)MN;
+    const float4 g = sum_parts(part + at, mn2, S), u = sum_parts(part + at + N, mn2, S);
+    uint2 o;
+    o.x = silu_mul_rounded_bits(g.x, u.x) | ((uint32_t)silu_mul_rounded_bits(g.y, u.y) << 16);
+    o.y = silu_mul_rounded_bits(g.z, u.z) | ((uint32_t)silu_mul_rounded_bits(g.w, u.w) << 16);
     *reinterpret_cast<uint2*>(Y + i) = o;
 }
 
@@ -985,9 +857,8 @@ __global__ __launch_bounds__(512) void stream_gemm_kernel(const uint16_t* __rest
 // activation and scale loads, 8-byte zero-point loads; and at least 128 workgroups.
 bool stream_shape(int FMT, int M, int K, int N, const void* x, const void* qw, const void* sc, const void* zp,
                   const void* y) {
-    // up to 32 tokens for INT4 and 16 for e4m3 it is faster on MI355X than the tiles (measured at
-    // K = N = 4096: INT4 M = 32 11.9 vs 12.8 us, M = 64 18.8 vs 16.9 us; e4m3 M = 64 19.8 vs 13.3 us):
-    // every workgroup reads all M x K activations, which outweighs the weight stream as M grows
+    // up to 32 tokens for INT4 and 16 for e4m3: every workgroup reads all M x K activations, which
+    // outweighs the weight stream as M grows (stream_better says where it wins against the wide tile)
     if (M < 1 || M > (FMT == kInt4G32 ? 32 : 16) || N % 4 || N < 128 * kStreamRows) return false;
     if (!(MOSS_ALIGNED(x, 16) && MOSS_ALIGNED(qw, 16) && MOSS_ALIGNED(y, 8))) return false;
     if (K % 4096) return false;  // K / 256 groups per wave: whole 4-quad steps
@@ -1008,7 +879,7 @@ void launch_stream(const void* x, const void* qw, const void* sc, const void* zp
 
 struct Plan {
     int bm, bn, split;
-    bool reg;  // the register-weight 128 x 128 INT4 tile
+    bool reg;  // the 128 x 128 INT4 copy tile
 };
 
 // Shapes the register-weight tile takes: whole blocks of kTs steps, 4-output stores, and for
@@ -1019,7 +890,8 @@ bool reg_tile_shape(int K, int N, bool int4) {
     return int4 && N % 4 == 0 && (K / kBK) % kTs == 0 && G % 16 == 0 && (G % 128) % 16 == 0;
 }
 
-// INT4: the register-weight tile, 32, 64 or 128 tokens deep.  M > 64 (MFMA-bound): split K (2..8,
+// The K split of the 128-token copy tile (bm: the token depth its split is counted with), which also
+// bounds the wide tile's above 64 tokens (wide_max_split).  M > 64 (MFMA-bound): split K (2..8,
 // >= 2 blocks each) while the doubled workgroup count still fits one per CU.  M <= 64 (bound by
 // the weight stream): split while the workgroups fit two per CU and the fp32 partials (written
 // and read back once) stay below half the weight bytes.  Shapes it does not take use the LDS
@@ -1049,6 +921,10 @@ Plan plan_gemm(int M, int K, int N, bool int4) {
             p.split *= 2;
         return p;
     }
+}
+
+int wide_max_split(int fmt, int M, int K, int N) {
+    return fmt == kInt4G32 && M > 64 && plan_gemm(M, K, N, true).split == 1 ? 1 : 16;
 }
 
 Plan plan_lds(int M, int K, int N) {
@@ -1092,27 +968,83 @@ void launch_tile(const Plan& p, const void* x, const void* qw, const void* sc, c
         launch_tile2<BM, BN, FMT, true>(p, x, qw, sc, zp, y, part, M, K, N, row_scale, st);
 }
 
-template <int JT>
-void launch_reg(const Plan& p, const void* x, const void* qw, const void* sc, const void* zp, void* y, void* ws,
-                int M, int K, int N, hipStream_t st) {
-    const dim3 grid((unsigned)(((M + 32 * JT - 1) / (32 * JT)) * ((N + 127) / 128)), (unsigned)p.split);
-    if constexpr (JT == 4) {
-        if (p.split > 1)
-            hipLaunchKernelGGL((w4g32_gemm_tdma_kernel<true>), grid, dim3(256), 0, st, (const uint16_t*)x,
-                               (const uint4*)qw, (const uint16_t*)sc, (const uint8_t*)zp, (uint16_t*)y, (float*)ws, M, N, K,
-                               QkRope{});
-        else
-            hipLaunchKernelGGL((w4g32_gemm_tdma_kernel<false>), grid, dim3(256), 0, st, (const uint16_t*)x,
-                               (const uint4*)qw, (const uint16_t*)sc, (const uint8_t*)zp, (uint16_t*)y, (float*)ws, M, N, K,
-                               QkRope{});
-        return;
-    }
+void launch_copy_tile(const Plan& p, const void* x, const void* qw, const void* sc, const void* zp, void* y, void* ws,
+                      int M, int K, int N, hipStream_t st) {
+    const dim3 grid((unsigned)(((M + 127) / 128) * ((N + 127) / 128)), (unsigned)p.split);
     if (p.split > 1)
-        hipLaunchKernelGGL((w4g32_gemm_t_kernel<JT, true>), grid, dim3(256), 0, st, (const uint16_t*)x,
-                           (const uint4*)qw, (const uint16_t*)sc, (const uint8_t*)zp, (uint16_t*)y, (float*)ws, M, N, K);
+        hipLaunchKernelGGL((w4g32_gemm_tdma_kernel<true>), grid, dim3(256), 0, st, (const uint16_t*)x, (const uint4*)qw,
+                           (const uint16_t*)sc, (const uint8_t*)zp, (uint16_t*)y, (float*)ws, M, N, K, QkRope{});
     else
-        hipLaunchKernelGGL((w4g32_gemm_t_kernel<JT, false>), grid, dim3(256), 0, st, (const uint16_t*)x,
-                           (const uint4*)qw, (const uint16_t*)sc, (const uint8_t*)zp, (uint16_t*)y, (float*)ws, M, N, K);
+        hipLaunchKernelGGL((w4g32_gemm_tdma_kernel<false>), grid, dim3(256), 0, st, (const uint16_t*)x,
+                           (const uint4*)qw, (const uint16_t*)sc, (const uint8_t*)zp, (uint16_t*)y, (float*)ws, M, N, K,
+                           QkRope{});
+}
+
+// INT4, 2 to 4 tokens: the exact GEMV holding every token's x in registers reads the weights
+// once, on the VALU, each row of y equal to the single-token GEMV of its token.  Faster than the
+// weight-streaming kernel (measured on MI355X, 2 / 3 / 4 tokens: K = 4096, N = 12288: 9.8 /
+// 11.6 / 13.7 against 14.6 / 15.1 / 15.6 us; N = 24576: 16.5 / 20.6 / 24.0 against 27.4 / 28.2
+// / 29.3 us; K = 12288, N = 4096: 9.9 / 13.1 against 13.0 / 13.3 us) except 4 tokens at
+// K > 4096 (15.2 against 13.7 us), which stays on the streaming kernel.
+bool tokens_gemv(int M, int K, const void* x, const void* qw) {
+    return w4g32_gemv_tokens_shape(M, K) && (M <= 3 || K <= 4096) && MOSS_ALIGNED(x, 16) && MOSS_ALIGNED(qw, 16);
+}
+
+void reduce_parts(const void* part, const float* row_scale, void* y, int M, int N, int split, hipStream_t st) {
+    const int mn = M * N;
+    hipLaunchKernelGGL(gemm_reduce, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, st, (const float*)part,
+                       row_scale, (uint16_t*)y, mn, N, split);
+}
+
+bool split_fits(int split, const void* ws, long long ws_bytes, const void* y, int M, int N) {
+    return split == 1 || (ws && ws_bytes >= (long long)split * M * N * 4 && MOSS_ALIGNED(ws, 16) && MOSS_ALIGNED(y, 8));
+}
+
+// Where the weight-streaming kernel, which never splits K over workgroups, still beats the wide tile with
+// its partial sums: at most 256 workgroups (N <= 4096) and few activations to read in each (INT4 K = N =
+// 4096: M = 5 6.4 against 7.8 us, 16 8.2 / 8.9, 24 10.4 / 9.9; N = 6144, M = 6 11.3 / 10.2; e4m3 M = 2 6.1 /
+// 8.3, 16 8.3 / 9.2; K = 12288, M = 4 13.2 / 13.6, 8 15.5 / 13.9), and for e4m3, whose tile has no fewer
+// bytes to hide its steps behind, very few tokens or very many rows (N = 12288: M = 3 12.7 / 15.0, 12 17.5 /
+// 15.1; N = 24576: M = 5 27.0 / 34.7, 12 32.8 / 34.7, 16 36.2 / 35.2).
+bool stream_better(int fmt, int M, int K, int N) {
+    const long long mk = (long long)M * K;
+    if (N <= 4096) return mk <= 16 * 4096;
+    return fmt == kFp8E4M3 && mk <= (N >= 16384 ? 12 : 5) * 4096;
+}
+
+// Whether the wide tile (gemm_wide_kernel.h) takes a call, and how.  Above 64 INT4 tokens it splits K
+// only where plan_gemm does: there the fused epilogues run without a workspace, and the plain GEMM
+// of the same shape sums in the same order.  A call whose planned split finds no workspace goes to the
+// weight-streaming kernel if that takes it (K = N = 4096, M = 24: 10 us against 24 us unsplit).
+bool choose_wide(int fmt, int M, int K, int N, const void* x, const void* qw, const void* sc, const void* zp,
+                 const void* y, const void* ws, long long ws_bytes, WidePlan& p) {
+    if (!wide_shape(fmt, K, N) || !MOSS_ALIGNED(y, 8)) return false;
+    if (fmt == kInt4G32 && !(MOSS_ALIGNED(sc, 16) && MOSS_ALIGNED(zp, 8))) return false;
+    if (stream_shape(fmt, M, K, N, x, qw, sc, zp, y) && stream_better(fmt, M, K, N)) return false;
+    p = wide_plan(fmt, M, K, N, wide_max_split(fmt, M, K, N));
+    if (split_fits(p.split, ws, ws_bytes, y, M, N)) return true;
+    if (stream_shape(fmt, M, K, N, x, qw, sc, zp, y)) return false;
+    p = wide_plan(fmt, M, K, N, 1);
+    return true;
+}
+
+// The LDS tiles, and the 128-token copy tile for INT4 weights past the wide tile's 32-bit offsets;
+// returns the K split whose partials it left in ws (1: y holds the product).
+template <int FMT>
+int launch_tiles(const void* x, const void* qw, const void* sc, const void* zp, void* y, int M, int K, int N,
+                 const float* row_scale, void* ws, long long ws_bytes, hipStream_t st) {
+    Plan p = plan_gemm(M, K, N, FMT == kInt4G32);
+    // the register-weight tile stores 4 outputs (8 bytes) at a time and loads scales and zero
+    // bytes 16 and 8 at a time
+    if (p.reg && !(MOSS_ALIGNED(y, 8) && MOSS_ALIGNED(sc, 16) && MOSS_ALIGNED(zp, 8)))
+        p = plan_lds(M, K, N);
+    if (!split_fits(p.split, ws, ws_bytes, y, M, N)) p.split = 1;
+    if (p.reg) launch_copy_tile(p, x, qw, sc, zp, y, ws, M, K, N, st);
+    else if (p.bm == 64 && p.bn == 64) launch_tile<64, 64, FMT>(p, x, qw, sc, zp, y, ws, M, K, N, row_scale, st);
+    else if (p.bm == 64) launch_tile<64, 128, FMT>(p, x, qw, sc, zp, y, ws, M, K, N, row_scale, st);
+    else if (p.bn == 64) launch_tile<128, 64, FMT>(p, x, qw, sc, zp, y, ws, M, K, N, row_scale, st);
+    else launch_tile<128, 128, FMT>(p, x, qw, sc, zp, y, ws, M, K, N, row_scale, st);
+    return p.split;
 }
 
 // split_out: when non-null, a K-split plan leaves its fp32 partials in ws for the caller to reduce
@@ -1121,41 +1053,24 @@ template <int FMT>
 int launch_gemm(const void* x, const void* qw, const void* sc, const void* zp, void* y, int M, int K, int N,
                 const float* row_scale, void* ws, long long ws_bytes, hipStream_t st, int* split_out = nullptr) {
     if (split_out) *split_out = 1;
-    // INT4, 2 to 4 tokens: the exact GEMV holding every token's x in registers reads the weights
-    // once, on the VALU, each row of y equal to the single-token GEMV of its token.  Faster than the
-    // weight-streaming kernel (measured on MI355X, 2 / 3 / 4 tokens: K = 4096, N = 12288: 9.8 /
-    // 11.6 / 13.7 against 14.6 / 15.1 / 15.6 us; N = 24576: 16.5 / 20.6 / 24.0 against 27.4 / 28.2
-    // / 29.3 us; K = 12288, N = 4096: 9.9 / 13.1 against 13.0 / 13.3 us) except 4 tokens at
-    // K > 4096 (15.2 against 13.7 us), which stays on the streaming kernel.
-    if (FMT == kInt4G32 && w4g32_gemv_tokens_shape(M, K) && (M <= 3 || K <= 4096) && MOSS_ALIGNED(x, 16) &&
-        MOSS_ALIGNED(qw, 16))
+    if (FMT == kInt4G32 && tokens_gemv(M, K, x, qw))
         return w4g32_gemv_tokens_launch(x, qw, sc, zp, y, M, K, N, st);
-    if (stream_shape(FMT, M, K, N, x, qw, sc, zp, y)) {
+    int split = 1;
+    WidePlan wp;
+    if (choose_wide(FMT, M, K, N, x, qw, sc, zp, y, ws, ws_bytes, wp)) {
+        const WideArgs a{x, qw, sc, zp, row_scale, y, (float*)ws, M, K, N, QkRope{}};
+        const WideEpilogue epi = wp.split > 1 ? kWideSplit : kWidePlain;
+        if (int rc = FMT == kInt4G32 ? wide_launch_w4(epi, wp, a, st) : wide_launch_fp8(epi, wp, a, st)) return rc;
+        split = wp.split;
+    } else if (stream_shape(FMT, M, K, N, x, qw, sc, zp, y)) {
         launch_stream<FMT>(x, qw, sc, zp, row_scale, y, M, K, N, st);
-        return moss_launch_status();
+    } else {
+        split = launch_tiles<FMT>(x, qw, sc, zp, y, M, K, N, row_scale, ws, ws_bytes, st);
     }
-    Plan p = plan_gemm(M, K, N, FMT == kInt4G32);
-    // the register-weight tile stores 4 outputs (8 bytes) at a time and loads scales and zero
-    // bytes 16 and 8 at a time
-    if (p.reg && !(MOSS_ALIGNED(y, 8) && MOSS_ALIGNED(sc, 16) && MOSS_ALIGNED(zp, 8)))
-        p = plan_lds(M, K, N);
-    if (p.split > 1 &&
-        (!ws || ws_bytes < (long long)p.split * M * N * 4 || !MOSS_ALIGNED(ws, 16) || !MOSS_ALIGNED(y, 8)))
-        p.split = 1;
-    if (p.reg) {
-        if (p.bm == 32) launch_reg<1>(p, x, qw, sc, zp, y, ws, M, K, N, st);
-        else if (p.bm == 64) launch_reg<2>(p, x, qw, sc, zp, y, ws, M, K, N, st);
-        else launch_reg<4>(p, x, qw, sc, zp, y, ws, M, K, N, st);
-    } else if (p.bm == 64 && p.bn == 64) launch_tile<64, 64, FMT>(p, x, qw, sc, zp, y, ws, M, K, N, row_scale, st);
-    else if (p.bm == 64) launch_tile<64, 128, FMT>(p, x, qw, sc, zp, y, ws, M, K, N, row_scale, st);
-    else if (p.bn == 64) launch_tile<128, 64, FMT>(p, x, qw, sc, zp, y, ws, M, K, N, row_scale, st);
-    else launch_tile<128, 128, FMT>(p, x, qw, sc, zp, y, ws, M, K, N, row_scale, st);
-    if (p.split > 1 && split_out) {
-        *split_out = p.split;
-    } else if (p.split > 1) {
-        const int mn = M * N;
-        hipLaunchKernelGGL(gemm_reduce, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, st, (const float*)ws,
-                           FMT == kFp8E4M3 ? row_scale : nullptr, (uint16_t*)y, mn, N, p.split);
+    if (split > 1 && split_out) {
+        *split_out = split;
+    } else if (split > 1) {
+        reduce_parts(ws, FMT == kFp8E4M3 ? row_scale : nullptr, y, M, N, split, st);
     }
     return moss_launch_status();
 }
@@ -1187,11 +1102,16 @@ bool qk_rope_fusable_shape(int M, int K) {
     return p.reg && p.bm == 128 && p.split == 1;
 }
 
-// One workspace serves both formats and the LDS-tile fallback: the largest plan's partial sums.
+// One workspace serves both formats and every fallback: the largest plan's partial sums.
 long long gemm_workspace_bytes(int M, int K, int N) {
     long long bytes = 0;
     for (const Plan& p : {plan_gemm(M, K, N, true), plan_gemm(M, K, N, false), plan_lds(M, K, N)})
         if (p.split > 1) bytes = std::max(bytes, (long long)p.split * M * N * 4);
+    for (int fmt : {(int)kInt4G32, (int)kFp8E4M3})
+        if (wide_shape(fmt, K, N)) {
+            const int split = wide_plan(fmt, M, K, N, wide_max_split(fmt, M, K, N)).split;
+            if (split > 1) bytes = std::max(bytes, (long long)split * M * N * 4);
+        }
     return bytes;
 }
 
@@ -1229,6 +1149,9 @@ MOSS_API int moss_w4g32_gemm_silu(const void* x, const void* qw, const void* sc,
     MOSS_CHECK_ARG(MOSS_ALIGNED(x, 16) && MOSS_ALIGNED(qw, 16) && workspace_bytes >= 0);
     hipStream_t st = (hipStream_t)stream;
     if (silu_fusable_shape(M, K, N) && MOSS_ALIGNED(y, 8) && MOSS_ALIGNED(sc, 16) && MOSS_ALIGNED(zp, 8)) {
+        if (wide_shape(kInt4G32, K, 2 * N))
+            return wide_launch_w4(kWideSilu, wide_plan(kInt4G32, M, K, 2 * N, 1),
+                                  WideArgs{x, qw, sc, zp, nullptr, y, nullptr, M, K, N, QkRope{}}, st);
         const dim3 grid((unsigned)(((M + 127) / 128) * ((N + 63) / 64)));
         hipLaunchKernelGGL((w4g32_gemm_tdma_kernel<false, true>), grid, dim3(256), 0, st, (const uint16_t*)x,
                            (const uint4*)qw, (const uint16_t*)sc, (const uint8_t*)zp, (uint16_t*)y, (float*)nullptr,
@@ -1238,9 +1161,22 @@ MOSS_API int moss_w4g32_gemm_silu(const void* x, const void* qw, const void* sc,
     const long long inter = align16((long long)M * 2 * N * 2);
     MOSS_CHECK_ARG(workspace && MOSS_ALIGNED(workspace, 16) && workspace_bytes >= inter);
     char* ws = (char*)workspace;
-    if (int rc = launch_gemm<kInt4G32>(x, qw, sc, zp, ws, M, K, 2 * N, nullptr, ws + inter, workspace_bytes - inter, st))
+    WidePlan wp;
+    if (!tokens_gemv(M, K, x, qw) && MOSS_ALIGNED(y, 8) &&
+        choose_wide(kInt4G32, M, K, 2 * N, x, qw, sc, zp, ws, ws + inter, workspace_bytes - inter, wp) && wp.split == 1)
+        return wide_launch_w4(kWideSilu, wp, WideArgs{x, qw, sc, zp, nullptr, y, nullptr, M, K, N, QkRope{}}, st);
+    int split = 1;
+    if (int rc = launch_gemm<kInt4G32>(x, qw, sc, zp, ws, M, K, 2 * N, nullptr, ws + inter, workspace_bytes - inter, st,
+                                       &split))
         return rc;
-    return moss_silu_mul(ws, y, M, N, stream);
+    if (split == 1 || !MOSS_ALIGNED(y, 8)) {
+        if (split > 1) reduce_parts(ws + inter, nullptr, ws, M, 2 * N, split, st);
+        return moss_silu_mul(ws, y, M, N, stream);
+    }
+    const int mn = M * N;
+    hipLaunchKernelGGL(gemm_reduce_silu, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, st,
+                       (const float*)(ws + inter), (uint16_t*)y, mn, N, split);
+    return moss_launch_status();
 }
 
 extern "C" int moss_rmsnorm(const void* x, const void* res, const void* w, void* sum_out, void* y, int rows, int n,
@@ -1271,6 +1207,9 @@ MOSS_API int moss_w4g32_gemm_qk_rope(const void* x, const void* qw, const void* 
         const QkRope qr{(const uint16_t*)q_weight, (const uint16_t*)k_weight, (const uint16_t*)cos,
                         (const uint16_t*)sin, (uint16_t*)k_cache, (uint16_t*)v_cache, (const int64_t*)positions, L,
                         eps};
+        if (wide_shape(kInt4G32, K, kQkvN))
+            return wide_launch_w4(kWideQkRope, wide_plan(kInt4G32, M, K, kQkvN, 1),
+                                  WideArgs{x, qw, sc, zp, nullptr, q_out, nullptr, M, K, kQkvN, qr}, st);
         const dim3 grid((unsigned)(((M + 127) / 128) * (kQkvN / 128)));
         hipLaunchKernelGGL((w4g32_gemm_tdma_kernel<false, false, true>), grid, dim3(256), 0, st, (const uint16_t*)x,
                            (const uint4*)qw, (const uint16_t*)sc, (const uint8_t*)zp, (uint16_t*)q_out,
