@@ -41,7 +41,6 @@ struct QkvArgs {
     float eps;
 };
 
-typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 constexpr int kWaveRows = kSplit / 4;  // cache rows per wave

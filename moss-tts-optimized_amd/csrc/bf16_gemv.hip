@@ -16,8 +16,6 @@
 namespace moss {
 namespace {
 
-typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-
 // KC = K / 512 chunks of 8 values per lane.  NORM as in norm_fused.h (0: x used as is).
 template <int KC, int R, int NORM>
 __global__ __launch_bounds__(256) void bf16_gemv_kernel(const uint16_t* __restrict__ x, const uint4* __restrict__ w,

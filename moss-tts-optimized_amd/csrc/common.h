@@ -64,6 +64,21 @@ __device__ __forceinline__ uint32_t zero_of_group(const uint8_t* __restrict__ zr
     return ((uint32_t)zrow[b] >> sh) & 15u;
 }
 
+// ---------------------------------------------------------------- buffer reads
+typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
+
+// A range of memory read by buffer instructions: bytes at or past `bytes` from `base` read as zero; soff is wave-uniform.
+struct Span {
+    const void* base;
+    uint32_t bytes;
+};
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t span_rsrc(const Span& s) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(s.base), 0, s.bytes, 0x00020000);
+}
+__device__ __forceinline__ u32x4_t load16(const Span& s, uint32_t voff, uint32_t soff) {
+    return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(span_rsrc(s), voff, soff, 0));
+}
+
 // ---------------------------------------------------------------- cross-lane sums
 template <int CTRL>
 __device__ __forceinline__ float dpp_move(float v) {

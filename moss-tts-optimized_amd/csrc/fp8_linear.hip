@@ -24,8 +24,6 @@ int fp8_gemm_launch(const void* x, const void* w, const float* row_scale, void* 
 
 namespace {
 
-typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-
 template <bool HI>
 __device__ __forceinline__ uint32_t fp8x2_bf16x2(uint32_t w) {
     return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, HI));

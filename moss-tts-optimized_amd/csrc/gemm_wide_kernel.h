@@ -36,7 +36,6 @@ namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
-typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kXcds = 8;
 constexpr int kStep = 64;   // K of one step
@@ -53,20 +52,9 @@ __device__ __forceinline__ uint32_t fp8x2_to_bf16x2(uint32_t w) {
     return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, 1.0f, HI));
 }
 
-// A range of memory read by buffer instructions: bytes at or past `bytes` from `base` read as zero; soff is wave-uniform.
-struct Span {
-    const void* base;
-    uint32_t bytes;
-};
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t span_rsrc(const Span& s) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(s.base), 0, s.bytes, 0x00020000);
-}
 // 16 bytes per lane straight to lds + 16 lane
 __device__ __forceinline__ void lds_copy16(const Span& s, uint16_t* lds, uint32_t voff, uint32_t soff) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(span_rsrc(s), lds, 16, voff, soff, 0, 0);
-}
-__device__ __forceinline__ u32x4_t load16(const Span& s, uint32_t voff, uint32_t soff) {
-    return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(span_rsrc(s), voff, soff, 0));
 }
 __device__ __forceinline__ uint2 load8(const Span& s, uint32_t voff, uint32_t soff) {
     return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(span_rsrc(s), voff, soff, 0));

@@ -10,12 +10,19 @@
 //
 // Tiling (flash-attention style, online softmax in fp32): one workgroup per (32-token query tile,
 // HPW query heads of one KV head), KS waves per head: wave (kq, hw) takes query head hw of the group
-// and the 32-key part kq of every block of 32 KS keys, so a block's keys are split over the KS waves
+// and part kq of every block of 32 SUB KS keys, so a block's keys are split over the KS waves
 // of a head and the serial chain of blocks is KS times shorter than one wave per head would make
-// it.  Shapes: 2 heads x 4 parts (128-key blocks) while 16 workgroups per 32 tokens fill at most
-// one per CU, else 4 heads x 2 parts (64-key blocks).  Tiles are issued longest first.
+// it.  Shapes: 2 heads x 4 parts of 32 keys while 16 workgroups per 32 tokens fill at most
+// one per CU, else 4 heads x 2 parts of 64 keys.  Tiles are issued longest first.
+// What bounds it: the vector work and the serial chain of a block (two waves a SIMD, S before the
+// softmax before P V).  Per 32 keys and wave that was about 220 VALU instructions to 16 MFMAs; now about 130:
+// the running reference of the softmax moves, and O^T is rescaled, only when a score passes it by 2^8;
+// the scale goes into the exponent's fma; masked blocks are a branch of their own; and rows past the
+// last visible key are zeros of the buffer reads, not branches around loads.  Two 32-key tiles a wave and
+// block halve the barriers and give S two independent MFMA chains.  2048 tokens: 117 -> 82 us (416 TFLOP/s),
+// 1024: 34.7 -> 26.0, 512: 14.7 -> 13.1, 150 after 600: 17.3 -> 15.2.
 // Every K/V block staged in LDS serves all waves.  Per block and wave:
-//   S^T = K Q^T   (32 keys x 32 queries, 8 v_mfma_f32_32x32x16_bf16): with this orientation each
+//   S^T = K Q^T   (per 32 keys x 32 queries 8 v_mfma_f32_32x32x16_bf16): with this orientation each
 //                 lane holds one query and 16 of its keys, so the row max and sum need one
 //                 exchange with the lane 32 away;
 //   O^T += V^T P^T (d x queries, 2 x 4 MFMAs): P (rounded to bf16) is the B operand straight from
@@ -40,13 +47,14 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 constexpr int kQH = 32, kKH = 8, kD = 128;
 constexpr int kBQ = 32;              // query tokens per workgroup
 constexpr int kKPad = kD + 8;        // K rows in LDS (bf16), padded
+constexpr float kSlack = 8.f;        // log2 a score may pass its query's reference by
 
-// Workgroup shape: HPW query heads of one KV head, KS waves per head, wave kq taking the 32-key
-// part kq of every block of 32 KS keys.
-template <int HPW, int KS>
+// Workgroup shape: HPW query heads of one KV head, KS waves per head, wave kq taking the 32 SUB-key
+// part kq of every block of 32 SUB KS keys.
+template <int HPW, int KS, int SUB>
 struct Tile {
     static constexpr int kWaves = HPW * KS, kThreads = 64 * kWaves;
-    static constexpr int kBK = 32 * KS;                            // keys per block
+    static constexpr int kBK = 32 * SUB * KS;                      // keys per block
     static constexpr int kKPT = 16 * kBK / kThreads;               // keys per thread in the K/V copy
     static constexpr int kVPad = kBK + 4;                          // V^T rows in LDS (bf16), padded
     static constexpr int kKBytes = kBK * kKPad * 2;
@@ -58,12 +66,10 @@ struct Tile {
     static_assert(kKPT == 2 || kKPT == 4, "K/V copy takes 2 or 4 keys per thread");
 };
 
-typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-
 // KPT keys per thread: thread (kg, dc) = (tid / 16, tid % 16) holds keys KPT kg .. + KPT - 1 of
-// the block at d 8 dc .. + 7.  Rows after `last` (the last key any query of the tile sees) are
-// zeros, not loads: they may lie past the cache or hold rows never written, and a P of 0 times a
-// NaN there would still poison O.
+// the block at d 8 dc .. + 7.  Rows after `last` (the last key any query of the tile sees) lie past
+// the spans and read as zeros: they may lie past the cache or hold rows never written, and a P of 0
+// times a NaN there would still poison O.
 template <int KPT>
 struct KvRegs {
     u32x4_t k[KPT];
@@ -71,16 +77,12 @@ struct KvRegs {
 };
 
 template <int KPT>
-__device__ __forceinline__ void load_kv(KvRegs<KPT>& r, const uint16_t* __restrict__ kc,
-                                        const uint16_t* __restrict__ vc, int key0, int last, int tid) {
-    const int dc = tid & 15, kg = tid >> 4;
+__device__ __forceinline__ void load_kv(KvRegs<KPT>& r, const Span& kc, const Span& vc, int key0, int tid) {
+    const uint32_t off = (uint32_t)((KPT * (tid >> 4)) * kD + 8 * (tid & 15)) * 2u, block = (uint32_t)key0 * kD * 2u;
 #pragma unroll
     for (int i = 0; i < KPT; ++i) {
-        const int key = key0 + KPT * kg + i;
-        const size_t off = (size_t)key * kD + 8 * dc;
-        const u32x4_t z = {0u, 0u, 0u, 0u};
-        r.k[i] = key <= last ? *reinterpret_cast<const u32x4_t*>(kc + off) : z;
-        r.v[i] = key <= last ? *reinterpret_cast<const u32x4_t*>(vc + off) : z;
+        r.k[i] = load16(kc, off + 2u * kD * i, block);
+        r.v[i] = load16(vc, off + 2u * kD * i, block);
     }
 }
 
@@ -116,11 +118,11 @@ __device__ __forceinline__ void store_kv(const KvRegs<KPT>& r, uint16_t (*ks)[kK
     }
 }
 
-template <int HPW, int KS>
+template <int HPW, int KS, int SUB>
 __global__ __launch_bounds__(64 * HPW * KS, 1) void prefill_attention_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
     const int64_t* __restrict__ start, uint16_t* __restrict__ out, int n, int L) {
-    using T = Tile<HPW, KS>;
+    using T = Tile<HPW, KS, SUB>;
     constexpr int KPT = T::kKPT, BK = T::kBK, VPAD = T::kVPad;
     // two K + V^T stages (block b in stage b % 2: one barrier per block), then the combine area
     __shared__ __attribute__((aligned(16))) unsigned char smem[T::kLds];
@@ -134,8 +136,8 @@ __global__ __launch_bounds__(64 * HPW * KS, 1) void prefill_attention_kernel(
     const int last = (int)p0 + min(t0 + kBQ - 1, n - 1);
     const int nblk = last / BK + 1;
     const int first_masked = ((int)p0 + t0) / BK;  // blocks before it hold no key after any query
-    const uint16_t* kc = k_cache + (size_t)kvh * L * kD;
-    const uint16_t* vc = v_cache + (size_t)kvh * L * kD;
+    const Span kc{k_cache + (size_t)kvh * L * kD, (uint32_t)(last + 1) * kD * 2u};
+    const Span vc{v_cache + (size_t)kvh * L * kD, (uint32_t)(last + 1) * kD * 2u};
     auto stage_k = [&](int s) { return reinterpret_cast<uint16_t(*)[kKPad]>(smem + s * T::kStage); };
     auto stage_v = [&](int s) { return reinterpret_cast<uint16_t(*)[VPAD]>(smem + s * T::kStage + T::kKBytes); };
 
@@ -155,60 +157,69 @@ __global__ __launch_bounds__(64 * HPW * KS, 1) void prefill_attention_kernel(
     const float c = 0.08838834764831845f * 1.4426950408889634f;  // 1/sqrt(128) * log2(e)
 
     KvRegs<KPT> kv;
-    load_kv<KPT>(kv, kc, vc, 0, last, tid);
+    load_kv<KPT>(kv, kc, vc, 0, tid);
     store_kv<KPT, VPAD>(kv, stage_k(0), stage_v(0), tid);
-    if (nblk > 1) load_kv<KPT>(kv, kc, vc, BK, last, tid);
+    if (nblk > 1) load_kv<KPT>(kv, kc, vc, BK, tid);
     for (int b = 0; b < nblk; ++b) {
         // block b is staged by every wave, and every wave is done with block b - 1's stage
         __syncthreads();
         const uint16_t(*ks)[kKPad] = stage_k(b & 1);
         const uint16_t(*vt)[VPAD] = stage_v(b & 1);
-        if (BK * b + 32 * kq <= last) {  // else every key of this wave's part is masked
-            // S^T for this wave's 32-key part of the block
-            f32x16_t s = {};
+        const int part = 32 * SUB * kq;      // this wave's keys of the block
+        if (BK * b + part <= last) {         // else every one of them is masked
+            // S^T, SUB tiles of 32 keys
+            f32x16_t s[SUB];
 #pragma unroll
-            for (int kk = 0; kk < 8; ++kk) {
-                const bf16x8_t kf = *reinterpret_cast<const bf16x8_t*>(&ks[32 * kq + ql][16 * kk + 8 * half]);
-                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[kk], s, 0, 0, 0);
-            }
-            // element e: key BK b + 32 kq + 8 (e / 4) + 4 half + e % 4, query ql
-            const bool mask = b >= first_masked;
-            float bmax = -INFINITY;
+            for (int i = 0; i < SUB; ++i) s[i] = f32x16_t{};
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                float v = s[e] * c;
-                if (mask) {
-                    const int key = BK * b + 32 * kq + 8 * (e >> 2) + 4 * half + (e & 3);
-                    v = key <= qpos ? v : -INFINITY;
+            for (int kk = 0; kk < 8; ++kk)
+#pragma unroll
+                for (int i = 0; i < SUB; ++i) {
+                    const bf16x8_t kf = *reinterpret_cast<const bf16x8_t*>(&ks[part + 32 * i + ql][16 * kk + 8 * half]);
+                    s[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[kk], s[i], 0, 0, 0);
                 }
-                s[e] = v;
-                bmax = fmaxf(bmax, v);
-            }
-            bmax = max_xor32(bmax);  // the other 32-lane half's keys of the same query rows
-            const float mn = fmaxf(m, bmax);
-            const float mr = mn == -INFINITY ? 0.f : mn;  // no key of this wave visible yet: nothing changes
-            const float alpha = __builtin_amdgcn_exp2f(m - mr);
-            m = mn;
-            float bsum = 0.f;
-            bf16x8_t pf[2];
+            // element e of tile i: key BK b + part + 32 i + 8 (e / 4) + 4 half + e % 4, query ql
+            if (b >= first_masked) {
 #pragma unroll
-            for (int u = 0; u < 2; ++u)
+                for (int i = 0; i < SUB; ++i)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const int key = BK * b + part + 32 * i + 8 * (e >> 2) + 4 * half + (e & 3);
+                        s[i][e] = key <= qpos ? s[i][e] : -INFINITY;
+                    }
+            }
+            float bmax = fmaxf(s[0][0], s[0][1]);
+#pragma unroll
+            for (int e = 2; e < 16 * SUB; e += 2) bmax = fmaxf(fmaxf(bmax, s[e >> 4][e & 15]), s[e >> 4][(e & 15) + 1]);
+            bmax = max_xor32(bmax) * c;  // with the other 32-lane half's keys of the same query rows
+            // the reference m only has to keep exp2(s c - m) in range: it moves up, and the sums with it,
+            // when some query of the wave passes it by 2^8 (its first visible key among them)
+            if (__any(bmax > m + kSlack)) {
+                const float mn = fmaxf(m, bmax);
+                const float alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+                m = mn;
+                l *= alpha;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) o[i][e] *= alpha;
+            }
+            const float mr = m == -INFINITY ? 0.f : m;  // no key of this wave visible yet: every P is 0
+            float bsum = 0.f;
+            bf16x8_t pf[2 * SUB];
+#pragma unroll
+            for (int u = 0; u < 2 * SUB; ++u)
 #pragma unroll
                 for (int v = 0; v < 8; ++v) {
-                    const float p = __builtin_amdgcn_exp2f(s[8 * u + v] - mr);
+                    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u >> 1][8 * (u & 1) + v], c, -mr));
                     bsum += p;
                     pf[u][v] = (__bf16)p;
                 }
-            bsum = sum_xor32(bsum);
-            l = l * alpha + bsum;
+            l += sum_xor32(bsum);
+            // O^T += V^T P^T: K step u covers keys part + 16 u + {4 half + 0..3, 8 + 4 half + 0..3}
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) o[i][e] *= alpha;
-            // O^T += V^T P^T: K step u covers keys 32 kq + 16 u + {4 half + 0..3, 8 + 4 half + 0..3}
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const int key = 32 * kq + 16 * u + 4 * half;
+            for (int u = 0; u < 2 * SUB; ++u) {
+                const int key = part + 16 * u + 4 * half;
 #pragma unroll
                 for (int dt = 0; dt < 4; ++dt) {
                     const uint16_t* row = vt[32 * dt + ql];
@@ -222,7 +233,7 @@ __global__ __launch_bounds__(64 * HPW * KS, 1) void prefill_attention_kernel(
         }
         if (b + 1 < nblk) {  // stage block b + 1 (its stage was last read for block b - 1)
             store_kv<KPT, VPAD>(kv, stage_k((b + 1) & 1), stage_v((b + 1) & 1), tid);
-            if (b + 2 < nblk) load_kv<KPT>(kv, kc, vc, BK * (b + 2), last, tid);
+            if (b + 2 < nblk) load_kv<KPT>(kv, kc, vc, BK * (b + 2), tid);
         }
     }
     // KS waves per head: each finishes the d tiles dt with dt % KS == kq, from every wave's O^T,
@@ -302,11 +313,11 @@ __global__ __launch_bounds__(64 * HPW * KS, 1) void prefill_attention_kernel(
     }
 }
 
-template <int HPW, int KS>
+template <int HPW, int KS, int SUB>
 void launch_prefill(const void* q, const void* k_cache, const void* v_cache, const void* start, void* out, int n,
                     int L, hipStream_t stream) {
     const dim3 grid((unsigned)((n + kBQ - 1) / kBQ), (unsigned)(kKH * (4 / HPW)));
-    hipLaunchKernelGGL((prefill_attention_kernel<HPW, KS>), grid, dim3(Tile<HPW, KS>::kThreads), 0, stream,
+    hipLaunchKernelGGL((prefill_attention_kernel<HPW, KS, SUB>), grid, dim3(Tile<HPW, KS, SUB>::kThreads), 0, stream,
                        (const uint16_t*)q, (const uint16_t*)k_cache, (const uint16_t*)v_cache,
                        (const int64_t*)start, (uint16_t*)out, n, L);
 }
@@ -326,10 +337,11 @@ MOSS_API int moss_prefill_attention(const void* q, const void* k_cache, const vo
     // workgroups per 32 tokens), then 4 heads x 2 key parts.  Measured on MI355X at start 0 (and
     // after a cached prefix), against 4 heads x 2 parts: 128 / 256 / 512 tokens in 7.4 / 9.5 /
     // 14.1 us against 9.3 / 12.2 / 18.9, 128 after 1900 rows in 34 against 53; 1024 and 2048 tokens
-    // in 31 / 106 us against 40 / 117 with 2 heads x 4 parts
+    // in 31 / 106 us against 40 / 117 with 2 heads x 4 parts (both with 32-key parts and the earlier
+    // softmax; today's times are at the head of this file)
     if (n <= 512)
-        launch_prefill<2, 4>(q, k_cache, v_cache, start, out, n, L, (hipStream_t)stream);
+        launch_prefill<2, 4, 1>(q, k_cache, v_cache, start, out, n, L, (hipStream_t)stream);
     else
-        launch_prefill<4, 2>(q, k_cache, v_cache, start, out, n, L, (hipStream_t)stream);
+        launch_prefill<4, 2, 2>(q, k_cache, v_cache, start, out, n, L, (hipStream_t)stream);
     return moss_launch_status();
 }

@@ -17,8 +17,6 @@ namespace {
 constexpr int kChunksPerThread = 4;
 constexpr long long kBytesPerWorkgroup = 256LL * 16 * kChunksPerThread;
 
-typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false);

@@ -24,8 +24,6 @@
 namespace moss {
 namespace {
 
-typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-
 __device__ __forceinline__ int dot4(uint32_t a, uint32_t b, int c) {
     return __builtin_amdgcn_sdot4((int)a, (int)b, c, false);
 }

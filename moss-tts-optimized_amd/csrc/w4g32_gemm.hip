@@ -48,8 +48,6 @@ constexpr int kXcds = 8;
 template <int BM, int BN>
 constexpr int stages_for() { return BM == 128 && BN == 128 ? 2 : 4; }
 
-typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-
 // Per-thread share of one K step: BM rows x 64 activations (BM / 32 x 16 B per thread) and one
 // piece of the BN x 64 weight tile.  The weight tile is 2 BN (row, 32-wide half) units; with
 // BN = 64 two threads share a unit (TPU = 2), each taking half of it.

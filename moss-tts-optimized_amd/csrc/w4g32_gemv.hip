@@ -196,8 +196,6 @@ __device__ __forceinline__ void rows_exact_from_lds(const uint16_t* xn, const Ro
     }
 }
 
-typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
-
 // Non-temporal loads: every weight byte is read once.
 template <int KG, bool FULL>
 __device__ __forceinline__ void load_row_nt(RowLoad<KG>& r, const uint4* __restrict__ qw,
