@@ -67,6 +67,12 @@ int moss_w4g32_quantize_minmax(const void *w, void *qw, void *sc, void *zp, int 
  * static_scales and the no-Hessian rounding of src/moss_tts/_runtime/calibrated_quant.py:36-38,74-77. */
 int moss_w4g32_quantize_symmetric(const void *w, void *qw, void *sc, void *zp, int K, int N, void *stream);
 
+/* Either quantizer with a range check: bad (a uint32 the device can write, pinned host memory for one)
+ * becomes 1 when some scale is not finite or reaches 2^120 (past which the decode and prefill kernels'
+ * in-register dequant overflows), and is left alone otherwise. */
+int moss_w4g32_quantize_checked(const void *w, void *qw, void *sc, void *zp, void *bad, int K, int N,
+                                int symmetric, void *stream);
+
 /* ------------------------------------------------------------ decode GEMV */
 /* dequant_mode of the decode GEMVs:
  *   MOSS_DEQUANT_EXACT (0)      every weight is the bit-exact bf16 dequant bf16_rne((q-z)*s)

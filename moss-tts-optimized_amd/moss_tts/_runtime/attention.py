@@ -40,7 +40,8 @@ def decode_attention(q: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, 
     ``[1, 1, 4096]``."""
     _cuda_contig("q", q, torch.bfloat16)
     dev = q.device
-    _require(q.numel() == QH * HD, f"q must hold {QH}x{HD} values")
+    if not (q.numel() == QH * HD):
+        raise ValueError(f"q must hold {QH}x{HD} values")
     for name, t in (("keys", keys), ("values", values)):
         _cuda_contig(name, t, torch.bfloat16, dev)
     _require(keys.shape == values.shape and keys.ndim == 4 and tuple(keys.shape[:2]) == (1, KH)
@@ -81,10 +82,12 @@ def decode_attention_qkv(qkv: torch.Tensor, q_norm: torch.Tensor, k_norm: torch.
     _require(L % 64 == 0 and L <= 32768, "the cache length must be a multiple of 64, at most 32768")
     for name, t in (("q_norm", q_norm), ("k_norm", k_norm)):
         _cuda_contig(name, t, torch.bfloat16, dev)
-        _require(t.numel() == HD, f"{name} must hold {HD} values")
+        if not (t.numel() == HD):
+            raise ValueError(f"{name} must hold {HD} values")
     for name, t in (("cos", cos), ("sin", sin)):
         _cuda_contig(name, t, torch.bfloat16, dev)
-        _require(t.numel() == L * HD, f"{name} must be an [L, {HD}] table")
+        if not (t.numel() == L * HD):
+            raise ValueError(f"{name} must be an [L, {HD}] table")
     _cuda_contig("position", position, torch.int64, dev)
     _require(position.numel() == 1, "one int64 position required")
     _require(_aligned(keys, 16) and _aligned(values, 16), "KV buffers must be 16-byte aligned")
@@ -94,7 +97,8 @@ def decode_attention_qkv(qkv: torch.Tensor, q_norm: torch.Tensor, k_norm: torch.
         out = torch.empty((1, 1, QH * HD), device=dev, dtype=torch.bfloat16)
     else:
         _cuda_contig("out", out, torch.bfloat16, dev)
-        _require(out.numel() == QH * HD, f"out must hold {QH * HD} values")
+        if not (out.numel() == QH * HD):
+            raise ValueError(f"out must hold {QH * HD} values")
     if not quantize:
         _require(out_activation is None, "out_activation needs quantize=True")
         native.call("moss_decode_attention_qkv", native.ptr(qkv), native.ptr(q_norm), native.ptr(k_norm),
@@ -118,7 +122,8 @@ def prefill_attention(q: torch.Tensor, keys: torch.Tensor, values: torch.Tensor,
     ``[n, 4096]``."""
     _cuda_contig("q", q, torch.bfloat16)
     dev = q.device
-    _require(q.numel() % (QH * HD) == 0 and q.numel() > 0, f"q must hold n x {QH} x {HD} values")
+    if not (q.numel() % (QH * HD) == 0 and q.numel() > 0):
+        raise ValueError(f"q must hold n x {QH} x {HD} values")
     n = q.numel() // (QH * HD)
     for name, t in (("keys", keys), ("values", values)):
         _cuda_contig(name, t, torch.bfloat16, dev)
@@ -134,7 +139,8 @@ def prefill_attention(q: torch.Tensor, keys: torch.Tensor, values: torch.Tensor,
         out = torch.empty((n, QH * HD), device=dev, dtype=torch.bfloat16)
     else:
         _cuda_contig("out", out, torch.bfloat16, dev)
-        _require(out.numel() == n * QH * HD, f"out must hold {n * QH * HD} values")
+        if not (out.numel() == n * QH * HD):
+            raise ValueError(f"out must hold {n * QH * HD} values")
     native.call("moss_prefill_attention", native.ptr(q), native.ptr(keys), native.ptr(values), native.ptr(start),
                 native.ptr(out), n, L, native.stream_of(q))
     return out
@@ -149,7 +155,8 @@ def embedding_sum(ids: torch.Tensor, text_weight: torch.Tensor, audio_weight: to
     _cuda_contig("audio_weight", audio_weight, torch.bfloat16, dev)
     _require(text_weight.ndim == 2 and audio_weight.ndim == 3, "text [V, H] and audio [Q, V, H] tables required")
     q = audio_weight.shape[0]
-    _require(ids.shape[-1] == q + 1, f"ids must end in a dimension of {q + 1}")
+    if not (ids.shape[-1] == q + 1):
+        raise ValueError(f"ids must end in a dimension of {q + 1}")
     h = text_weight.shape[1]
     _require(audio_weight.shape[2] == h, "text and audio widths differ")
     t = ids.numel() // (q + 1)

@@ -43,10 +43,14 @@ class QuantLinearG32(nn.Module):
         (``src/moss_tts/_runtime/calibrated_quant.py:36-38,74-77``)."""
         _require(weight.is_cuda and weight.ndim == 2, "a 2-D device weight [out, in] is required")
         w = weight.detach().float().contiguous()
-        return cls(w4g32.quantize_symmetric(w) if symmetric else w4g32.quantize_minmax(w), **kw)
+        packed, check = w4g32.quantize_launch(w, symmetric)
+        module = cls(packed, **kw)
+        check()  # after the module is made: the device quantizes meanwhile
+        return module
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        _require(x.shape[-1] == self.in_features, f"expected {self.in_features} input features")
+        if not (x.shape[-1] == self.in_features):
+            raise ValueError(f"expected {self.in_features} input features")
         rows = x.numel() // self.in_features
         if rows == 1:
             return w4g32.gemv(x.contiguous(), self.packed, dequant=self.dequant)
@@ -62,10 +66,13 @@ class QuantGateUpG32(QuantLinearG32):
     epilogue ``src/moss_tts/_runtime/dp4a_scaled.py:64-68``)."""
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        _require(x.shape[-1] == self.in_features, f"expected {self.in_features} input features")
+        if not (x.shape[-1] == self.in_features):
+            raise ValueError(f"expected {self.in_features} input features")
         rows = x.numel() // self.in_features
         if rows == 1:
             return w4g32.gateup_silu(x.contiguous(), self.packed, dequant=self.dequant)
+        if self.out_features % 8 == 0:
+            return w4g32.gemm_silu(x.contiguous(), self.packed)
         from . import pointwise
 
         return pointwise.silu_mul(w4g32.gemm(x.contiguous(), self.packed))
@@ -89,7 +96,8 @@ class Bf16Linear(nn.Module):
         return self.weight.numel() * self.weight.element_size()
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        _require(x.shape[-1] == self.in_features, f"expected {self.in_features} input features")
+        if not (x.shape[-1] == self.in_features):
+            raise ValueError(f"expected {self.in_features} input features")
         _require(x.numel() == self.in_features, "the bf16 heads run on one row (the decode step's last token)")
         return bf16.gemv(x.contiguous(), self.weight)
 

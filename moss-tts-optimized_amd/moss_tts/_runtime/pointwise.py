@@ -18,7 +18,8 @@ def _norm_common(x: torch.Tensor, weight: torch.Tensor):
     _cuda_contig("x", x, torch.bfloat16)
     _cuda_contig("weight", weight, torch.bfloat16, x.device)
     n = x.shape[-1]
-    _require(weight.numel() == n, f"weight must have {n} values")
+    if not (weight.numel() == n):
+        raise ValueError(f"weight must have {n} values")
     _require(n % 8 == 0 and n <= 8192, "hidden size must be a multiple of 8 and <= 8192")
     _require(_aligned(x, 16) and _aligned(weight, 16), "x and weight must be 16-byte aligned")
     return n, x.numel() // n
@@ -62,16 +63,19 @@ def qk_rope(qkv: torch.Tensor, q_weight: torch.Tensor, k_weight: torch.Tensor, c
     ``n * 32 * 128`` values to write ``q`` into (``[1, n, 32, 128]`` order)."""
     _cuda_contig("qkv", qkv, torch.bfloat16)
     dev = qkv.device
-    _require(qkv.shape[-1] == QKV, f"Qwen3-8B QKV rows of {QKV} required")
+    if not (qkv.shape[-1] == QKV):
+        raise ValueError(f"Qwen3-8B QKV rows of {QKV} required")
     n = qkv.numel() // QKV
     L = keys.shape[2] if keys.ndim == 4 else 0
     for name, t in (("cos", cos), ("sin", sin)):
         _cuda_contig(name, t, torch.bfloat16, dev)
         rows = L if cos_by_position else n
-        _require(t.numel() == rows * HD, f"{name} must hold {rows} rows of {HD}")
+        if not (t.numel() == rows * HD):
+            raise ValueError(f"{name} must hold {rows} rows of {HD}")
     for name, t in (("q_weight", q_weight), ("k_weight", k_weight)):
         _cuda_contig(name, t, torch.bfloat16, dev)
-        _require(t.numel() == HD, f"{name} must hold {HD} values")
+        if not (t.numel() == HD):
+            raise ValueError(f"{name} must hold {HD} values")
     for name, t in (("keys", keys), ("values", values)):
         _cuda_contig(name, t, torch.bfloat16, dev)
     _require(keys.shape == values.shape and keys.ndim == 4 and tuple(keys.shape[:2]) == (1, KH)
@@ -81,7 +85,8 @@ def qk_rope(qkv: torch.Tensor, q_weight: torch.Tensor, k_weight: torch.Tensor, c
     _require(n <= L, "more tokens than KV rows")
     if out is not None:
         _cuda_contig("out", out, torch.bfloat16, dev)
-        _require(out.numel() == n * QH * HD, f"out must hold {n * QH * HD} values")
+        if not (out.numel() == n * QH * HD):
+            raise ValueError(f"out must hold {n * QH * HD} values")
         q = out.view(1, n, QH, HD)
     else:
         q = torch.empty((1, n, QH, HD), device=dev, dtype=torch.bfloat16)

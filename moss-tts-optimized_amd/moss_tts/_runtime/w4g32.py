@@ -23,12 +23,15 @@ def _require(cond: bool, msg: str) -> None:
 
 
 def _cuda_contig(name: str, t: torch.Tensor, dtype: torch.dtype, device=None) -> None:
+    # one test for the usual case: the messages below are formed only for the call that they refuse
+    if (isinstance(t, torch.Tensor) and t.dtype == dtype and t.is_cuda and t.is_contiguous()
+            and (device is None or t.device == device)):
+        return
     _require(isinstance(t, torch.Tensor), f"{name} must be a tensor")
     _require(t.dtype == dtype, f"{name} must be {dtype}, got {t.dtype}")
     _require(t.is_cuda, f"{name} must be a CUDA (HIP) tensor")
     _require(t.is_contiguous(), f"{name} must be contiguous")
-    if device is not None:
-        _require(t.device == device, f"{name} must be on {device}, got {t.device}")
+    _require(device is None or t.device == device, f"{name} must be on {device}, got {t.device}")
 
 
 def _aligned(t: torch.Tensor, a: int) -> bool:
@@ -42,11 +45,13 @@ def _aligned(t: torch.Tensor, a: int) -> bool:
 MAX_SCALE = 2.0 ** 120
 
 
+_SCALE_RANGE = "scales must be finite and below 2^120 in magnitude for the exact in-register dequant"
+
+
 def _check_scales(scales: torch.Tensor) -> None:
     """Raise unless every scale is finite and below :data:`MAX_SCALE` in magnitude (one reduction
     and one host sync, at load time)."""
-    _require(bool((scales.float().abs() < MAX_SCALE).all()),
-             "scales must be finite and below 2^120 in magnitude for the exact in-register dequant")
+    _require(bool((scales.float().abs() < MAX_SCALE).all()), _SCALE_RANGE)
 
 
 @dataclass(frozen=True)
@@ -63,14 +68,17 @@ class PackedW4G32:
     def __post_init__(self):
         qw, sc, zp = self.qw, self.scales, self.zeros
         _cuda_contig("qw", qw, torch.int32)
-        _cuda_contig("scales", sc, torch.bfloat16, qw.device)
-        _cuda_contig("zeros", zp, torch.uint8, qw.device)
+        dev = qw.device
+        _cuda_contig("scales", sc, torch.bfloat16, dev)
+        _cuda_contig("zeros", zp, torch.uint8, dev)
         _require(qw.ndim == 2 and sc.ndim == 2 and zp.ndim == 2, "packed tensors must be 2-D")
         n, k8 = qw.shape
         k = 8 * k8
         _require(k % 64 == 0, "K must be a multiple of 64")
-        _require(tuple(sc.shape) == (n, k // GROUP), f"scales must be [{n}, {k // GROUP}], got {tuple(sc.shape)}")
-        _require(tuple(zp.shape) == (n, k // 64), f"zeros must be [{n}, {k // 64}], got {tuple(zp.shape)}")
+        if sc.shape != (n, k // GROUP):
+            raise ValueError(f"scales must be [{n}, {k // GROUP}], got {tuple(sc.shape)}")
+        if zp.shape != (n, k // 64):
+            raise ValueError(f"zeros must be [{n}, {k // 64}], got {tuple(zp.shape)}")
         _require(_aligned(qw, 16), "qw must be 16-byte aligned")
 
     @property
@@ -119,8 +127,10 @@ def repack_gptq(qweight: torch.Tensor, scales: torch.Tensor, qzeros: torch.Tenso
     k8, n = qweight.shape
     k = 8 * k8
     _require(k % 64 == 0 and n % 8 == 0, "K must be a multiple of 64 and N of 8")
-    _require(tuple(scales.shape) == (k // GROUP, n), f"scales must be [{k // GROUP}, {n}]")
-    _require(tuple(qzeros.shape) == (k // GROUP, n // 8), f"qzeros must be [{k // GROUP}, {n // 8}]")
+    if not (tuple(scales.shape) == (k // GROUP, n)):
+        raise ValueError(f"scales must be [{k // GROUP}, {n}]")
+    if not (tuple(qzeros.shape) == (k // GROUP, n // 8)):
+        raise ValueError(f"qzeros must be [{k // GROUP}, {n // 8}]")
     _check_scales(scales)
     out = PackedW4G32.empty(n, k, dev)
     native.call("moss_w4g32_repack_gptq", native.ptr(qweight), native.ptr(scales), native.ptr(qzeros),
@@ -140,7 +150,8 @@ def import_signed(packed: torch.Tensor, scales: torch.Tensor) -> PackedW4G32:
     n, k2 = packed.shape
     k = 2 * k2
     _require(k % 64 == 0, "K must be a multiple of 64")
-    _require(tuple(scales.shape) == (n, k // GROUP), f"scales must be [{n}, {k // GROUP}]")
+    if not (tuple(scales.shape) == (n, k // GROUP)):
+        raise ValueError(f"scales must be [{n}, {k // GROUP}]")
     sc = scales.to(torch.bfloat16).contiguous()
     if scales.dtype != torch.bfloat16:
         # the reference's own exactness rule before narrowing scale storage
@@ -155,32 +166,43 @@ def import_signed(packed: torch.Tensor, scales: torch.Tensor) -> PackedW4G32:
     return PackedW4G32(qw, sc, zp)
 
 
-def quantize_minmax(w: torch.Tensor) -> PackedW4G32:
-    """fp32 ``[N, K]`` -> :class:`PackedW4G32` (asymmetric min-max RTN per (row, 32-group))."""
+def quantize_launch(w: torch.Tensor, symmetric: bool):
+    """Launches a quantizer; returns the weight and the check to call before using it, which waits for the
+    stream and raises unless every scale is in range.  The kernel sets a host flag where a scale is formed."""
     _cuda_contig("w", w, torch.float32)
     _require(w.ndim == 2 and w.shape[1] % 64 == 0, "w must be [N, K] with K % 64 == 0")
     _require(_aligned(w, 16), "w must be 16-byte aligned")
     n, k = w.shape
     out = PackedW4G32.empty(n, k, w.device)
-    native.call("moss_w4g32_quantize_minmax", native.ptr(w), native.ptr(out.qw), native.ptr(out.scales),
-                native.ptr(out.zeros), k, n, native.stream_of(w))
-    _check_scales(out.scales)
+    bad = torch.empty(1, dtype=torch.int32, pin_memory=True)
+    bad[0] = 0
+    stream = torch.cuda.current_stream(w.device)
+    native.call("moss_w4g32_quantize_checked", native.ptr(w), native.ptr(out.qw), native.ptr(out.scales),
+                native.ptr(out.zeros), native.ptr(bad), k, n, int(symmetric), stream.cuda_stream)
+
+    def check() -> None:
+        stream.synchronize()
+        _require(bad.item() == 0, _SCALE_RANGE)
+
+    return out, check
+
+
+def _quantize(w: torch.Tensor, symmetric: bool) -> PackedW4G32:
+    out, check = quantize_launch(w, symmetric)
+    check()
     return out
+
+
+def quantize_minmax(w: torch.Tensor) -> PackedW4G32:
+    """fp32 ``[N, K]`` -> :class:`PackedW4G32` (asymmetric min-max RTN per (row, 32-group))."""
+    return _quantize(w, False)
 
 
 def quantize_symmetric(w: torch.Tensor) -> PackedW4G32:
     """fp32 ``[N, K]`` -> :class:`PackedW4G32` with the reference's static symmetric scales
     (``bf16(max|w_g| / 7)``) and round-to-nearest codes in [-7, 7], stored with zero point 8
     (``src/moss_tts/_runtime/calibrated_quant.py:36-38,74-77``)."""
-    _cuda_contig("w", w, torch.float32)
-    _require(w.ndim == 2 and w.shape[1] % 64 == 0, "w must be [N, K] with K % 64 == 0")
-    _require(_aligned(w, 16), "w must be 16-byte aligned")
-    n, k = w.shape
-    out = PackedW4G32.empty(n, k, w.device)
-    native.call("moss_w4g32_quantize_symmetric", native.ptr(w), native.ptr(out.qw), native.ptr(out.scales),
-                native.ptr(out.zeros), k, n, native.stream_of(w))
-    _check_scales(out.scales)
-    return out
+    return _quantize(w, True)
 
 
 def unpack_codes(w: PackedW4G32) -> torch.Tensor:
@@ -205,8 +227,10 @@ _MAX_GEMV_K = 8 * 64 * 32
 
 def _check_row(x: torch.Tensor, w: PackedW4G32) -> None:
     _cuda_contig("x", x, torch.bfloat16, w.device)
-    _require(x.numel() == w.K, f"one contiguous bf16 row of {w.K} values required, got shape {tuple(x.shape)}")
-    _require(w.K <= _MAX_GEMV_K, f"decode GEMV supports K <= {_MAX_GEMV_K}")
+    if not (x.numel() == w.K):
+        raise ValueError(f"one contiguous bf16 row of {w.K} values required, got shape {tuple(x.shape)}")
+    if not (w.K <= _MAX_GEMV_K):
+        raise ValueError(f"decode GEMV supports K <= {_MAX_GEMV_K}")
     _require(_aligned(x, 16), "x must be 16-byte aligned")
 
 
@@ -238,7 +262,8 @@ def gemv(x: torch.Tensor, w: PackedW4G32, *, rows_per_wave: int = 0, dequant: in
     m = x.numel() // w.K if w.K else 0
     _require(x.shape[-1] == w.K and m * w.K == x.numel() and 1 <= m <= MAX_GEMV_TOKENS,
              f"1 to {MAX_GEMV_TOKENS} contiguous bf16 rows of {w.K} values required, got shape {tuple(x.shape)}")
-    _require(w.K <= _MAX_GEMV_K, f"decode GEMV supports K <= {_MAX_GEMV_K}")
+    if not (w.K <= _MAX_GEMV_K):
+        raise ValueError(f"decode GEMV supports K <= {_MAX_GEMV_K}")
     _require(_aligned(x, 16), "x must be 16-byte aligned")
     rows = _rows_arg(rows_per_wave)
     mode = _mode_arg(dequant)
@@ -270,20 +295,23 @@ def _norm_call(name, x, norm_weight, eps, w, n_out, residual, rows_per_wave, deq
     _check_row(x, w)
     _require(w.K % 2048 == 0 and w.K <= 8192, "the fused norm needs K % 2048 == 0 and K <= 8192")
     _cuda_contig("norm_weight", norm_weight, torch.bfloat16, w.device)
-    _require(norm_weight.numel() == w.K, f"norm_weight must hold {w.K} values")
+    if not (norm_weight.numel() == w.K):
+        raise ValueError(f"norm_weight must hold {w.K} values")
     _require(_aligned(norm_weight, 16), "norm_weight must be 16-byte aligned")
     rows = _rows_arg(rows_per_wave)
     mode = _mode_arg(dequant)
     summed = None
     if residual is not None:
         _cuda_contig("residual", residual, torch.bfloat16, w.device)
-        _require(residual.numel() == w.K and _aligned(residual, 16), f"residual must be an aligned row of {w.K}")
+        if not (residual.numel() == w.K and _aligned(residual, 16)):
+            raise ValueError(f"residual must be an aligned row of {w.K}")
         summed = torch.empty_like(x)
     if out is None:
         y = torch.empty((*x.shape[:-1], n_out), dtype=torch.bfloat16, device=x.device)
     else:
         _cuda_contig("out", out, torch.bfloat16, w.device)
-        _require(out.numel() == n_out, f"out must hold {n_out} values")
+        if not (out.numel() == n_out):
+            raise ValueError(f"out must hold {n_out} values")
         y = out
     native.call(name, native.ptr(x), native.ptr(residual) if residual is not None else None, native.ptr(norm_weight),
                 native.ptr(summed) if summed is not None else None, float(eps), native.ptr(w.qw),
@@ -313,7 +341,8 @@ def gemm(x: torch.Tensor, w: PackedW4G32) -> torch.Tensor:
     """Prefill projection: bf16 ``[..., M, K]`` -> bf16 ``[..., M, N]`` on the matrix cores, with
     bit-exact bf16 dequantized weights and fp32 accumulation."""
     _cuda_contig("x", x, torch.bfloat16, w.device)
-    _require(x.shape[-1] == w.K, f"x must end in a dimension of {w.K}")
+    if not (x.shape[-1] == w.K):
+        raise ValueError(f"x must end in a dimension of {w.K}")
     _require(_aligned(x, 16), "x must be 16-byte aligned")
     m = x.numel() // w.K
     _require(m > 0, "empty input")
@@ -329,7 +358,8 @@ def gemm_silu(x: torch.Tensor, w: PackedW4G32) -> torch.Tensor:
     bf16 ``[..., M, K]`` -> bf16 ``[..., M, N]``, equal bit for bit to ``silu_mul(gemm(x, w))``
     (``src/moss_tts/_runtime/llm.py:27-29``, ``prefill_pointwise.py:18-31``)."""
     _cuda_contig("x", x, torch.bfloat16, w.device)
-    _require(x.shape[-1] == w.K, f"x must end in a dimension of {w.K}")
+    if not (x.shape[-1] == w.K):
+        raise ValueError(f"x must end in a dimension of {w.K}")
     _require(_aligned(x, 16), "x must be 16-byte aligned")
     _require(w.N % 8 == 0, "gate||up weight needs 2 N rows with N % 4 == 0")
     m, n = x.numel() // w.K, w.N // 2
@@ -353,9 +383,11 @@ def gemm_qk_rope(x: torch.Tensor, w: PackedW4G32, q_weight: torch.Tensor, k_weig
     from . import pointwise
 
     _cuda_contig("x", x, torch.bfloat16, w.device)
-    _require(x.shape[-1] == w.K, f"x must end in a dimension of {w.K}")
+    if not (x.shape[-1] == w.K):
+        raise ValueError(f"x must end in a dimension of {w.K}")
     _require(_aligned(x, 16), "x must be 16-byte aligned")
-    _require(w.N == pointwise.QKV, f"the QKV weight must hold {pointwise.QKV} rows")
+    if not (w.N == pointwise.QKV):
+        raise ValueError(f"the QKV weight must hold {pointwise.QKV} rows")
     n = x.numel() // w.K
     _require(n > 0, "empty input")
     dev = x.device
@@ -365,17 +397,21 @@ def gemm_qk_rope(x: torch.Tensor, w: PackedW4G32, q_weight: torch.Tensor, k_weig
     for name, t in (("keys", keys), ("values", values), ("cos", cos), ("sin", sin), ("q_weight", q_weight),
                     ("k_weight", k_weight)):
         _cuda_contig(name, t, torch.bfloat16, dev)
-        _require(_aligned(t, 8), f"{name} must be 8-byte aligned")
+        if not (_aligned(t, 8)):
+            raise ValueError(f"{name} must be 8-byte aligned")
     for name, t in (("cos", cos), ("sin", sin)):
-        _require(t.numel() == L * pointwise.HD, f"{name} must hold {L} rows of {pointwise.HD}")
+        if not (t.numel() == L * pointwise.HD):
+            raise ValueError(f"{name} must hold {L} rows of {pointwise.HD}")
     for name, t in (("q_weight", q_weight), ("k_weight", k_weight)):
-        _require(t.numel() == pointwise.HD, f"{name} must hold {pointwise.HD} values")
+        if not (t.numel() == pointwise.HD):
+            raise ValueError(f"{name} must hold {pointwise.HD} values")
     _cuda_contig("positions", positions, torch.int64, dev)
     _require(positions.numel() == n, "one int64 position per token required")
     _require(n <= L, "more tokens than KV rows")
     if out is not None:
         _cuda_contig("out", out, torch.bfloat16, dev)
-        _require(out.numel() == n * pointwise.QH * pointwise.HD, f"out must hold {n * pointwise.QH * pointwise.HD} values")
+        if not (out.numel() == n * pointwise.QH * pointwise.HD):
+            raise ValueError(f"out must hold {n * pointwise.QH * pointwise.HD} values")
         q = out.view(1, n, pointwise.QH, pointwise.HD)
     else:
         q = torch.empty((1, n, pointwise.QH, pointwise.HD), device=dev, dtype=torch.bfloat16)
@@ -395,16 +431,20 @@ def gemm_add_rmsnorm(x: torch.Tensor, w: PackedW4G32, residual: torch.Tensor, no
     ``pointwise.add_rmsnorm(gemm(x, w), residual, norm_weight, eps)``; a K-split GEMM's partial sums
     are reduced inside the norm kernel (``src/moss_tts/_runtime/prefill_pointwise.py:46-57``)."""
     _cuda_contig("x", x, torch.bfloat16, w.device)
-    _require(x.shape[-1] == w.K, f"x must end in a dimension of {w.K}")
+    if not (x.shape[-1] == w.K):
+        raise ValueError(f"x must end in a dimension of {w.K}")
     m = x.numel() // w.K
     _require(m > 0, "empty input")
     _require(w.N % 8 == 0 and w.N <= 8192, "the norm needs N % 8 == 0 and N <= 8192")
     _cuda_contig("residual", residual, torch.bfloat16, w.device)
-    _require(residual.numel() == m * w.N, f"residual must hold {m} x {w.N} values")
+    if not (residual.numel() == m * w.N):
+        raise ValueError(f"residual must hold {m} x {w.N} values")
     _cuda_contig("norm_weight", norm_weight, torch.bfloat16, w.device)
-    _require(norm_weight.numel() == w.N, f"norm_weight must hold {w.N} values")
+    if not (norm_weight.numel() == w.N):
+        raise ValueError(f"norm_weight must hold {w.N} values")
     for name, t in (("x", x), ("residual", residual), ("norm_weight", norm_weight)):
-        _require(_aligned(t, 16), f"{name} must be 16-byte aligned")
+        if not (_aligned(t, 16)):
+            raise ValueError(f"{name} must be 16-byte aligned")
     summed = torch.empty((*x.shape[:-1], w.N), dtype=torch.bfloat16, device=x.device)
     y = torch.empty_like(summed)
     wp, wb, _keep = native.gemm_workspace(m, w.K, w.N, x.device)
@@ -423,12 +463,14 @@ def gemm_noalloc(x: torch.Tensor, w: PackedW4G32, out: torch.Tensor) -> torch.Te
     entry point: the K-split partials live in the library's own device array, so the call allocates
     nothing.  Calls that overlap on one device race on that array."""
     _cuda_contig("x", x, torch.bfloat16, w.device)
-    _require(x.shape[-1] == w.K, f"x must end in a dimension of {w.K}")
+    if not (x.shape[-1] == w.K):
+        raise ValueError(f"x must end in a dimension of {w.K}")
     _require(_aligned(x, 16), "x must be 16-byte aligned")
     m = x.numel() // w.K
     _require(m > 0, "empty input")
     _cuda_contig("out", out, torch.bfloat16, w.device)
-    _require(out.numel() == m * w.N, f"out must hold {m} x {w.N} values")
+    if not (out.numel() == m * w.N):
+        raise ValueError(f"out must hold {m} x {w.N} values")
     need = int(native.lib().moss_gemm_workspace_bytes(m, w.K, w.N))
     _require(need <= NOALLOC_SCRATCH_BYTES, f"this GEMM's partial sums ({need} B) exceed the "
              f"{NOALLOC_SCRATCH_BYTES} B scratch of the allocation-free entry point")
