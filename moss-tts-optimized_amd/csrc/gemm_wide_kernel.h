@@ -56,6 +56,12 @@ __device__ __forceinline__ uint32_t fp8x2_to_bf16x2(uint32_t w) {
 __device__ __forceinline__ void lds_copy16(const Span& s, uint16_t* lds, uint32_t voff, uint32_t soff) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(span_rsrc(s), lds, 16, voff, soff, 0, 0);
 }
+__device__ __forceinline__ uint32_t load_u16(const Span& s, uint32_t voff, uint32_t soff) {
+    return __builtin_amdgcn_raw_buffer_load_b16(span_rsrc(s), voff, soff, 0);
+}
+__device__ __forceinline__ uint32_t load_u8(const Span& s, uint32_t voff, uint32_t soff) {
+    return __builtin_amdgcn_raw_buffer_load_b8(span_rsrc(s), voff, soff, 0);
+}
 __device__ __forceinline__ uint2 load8(const Span& s, uint32_t voff, uint32_t soff) {
     return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(span_rsrc(s), voff, soff, 0));
 }
@@ -84,15 +90,17 @@ __device__ __forceinline__ uint32_t dequant_pair(uint32_t w, uint32_t mask, uint
 }
 
 
-template <int FMT, int R, int JT, int EPI>
+template <int FMT, int R, int JT, int EPI, bool ANY = false>
 __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
     const uint16_t* __restrict__ X, const uint8_t* qw, const uint16_t* sc, const uint8_t* zp,
     const float* __restrict__ row_scale, uint16_t* __restrict__ Y, float* __restrict__ part, int M, int N, int K,
     int split, QkRope qr) {
-    constexpr bool INT4 = FMT == kInt4G32;
+    static_assert(!ANY || EPI == kWidePlain || EPI == kWideSplit, "epilogues of whole heads and pairs");
+    constexpr bool INT4 = FMT == kInt4G32, SZ = INT4 && ANY;  // SZ: scale and zero loaded with each step's codes
     constexpr int BM = 32 * JT, BN = (EPI == kWideSilu ? 64 : 128) * R;
-    constexpr int W = 2;                // steps the codes travel ahead (divides kRing)
-    constexpr int CL = INT4 ? 1 : 2;    // code loads per row tile and step
+    constexpr int W = 2;                   // steps the codes travel ahead (divides kRing)
+    constexpr int CW = INT4 ? 1 : 2;        // code loads per row tile and step
+    constexpr int CL = SZ ? 3 : CW;         // weight loads per row tile and step
     constexpr int kTile = 2048 * JT;    // bf16 values of one step's activations
     __shared__ __attribute__((aligned(1024))) uint16_t X0[kTile];
     __shared__ __attribute__((aligned(1024))) uint16_t X1[kTile];
@@ -107,8 +115,15 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
     t /= mt;
     const int z = EPI == kWideSplit ? t % split : 0;
     const int n0 = (EPI == kWideSplit ? t / split : t) * BN;
-    const int G = K >> 5, steps = K / kStep / (EPI == kWideSplit ? split : 1);
+    const int G = K >> 5, total = K / kStep;
+    const int share = EPI == kWideSplit ? (ANY ? (total + split - 1) / split : total / split) : total;
+    const int steps = ANY ? (share + kRing - 1) & ~(kRing - 1) : share;
     const int kbase = z * steps * kStep;
+    // ANY: steps past the end of K read zeros, through empty spans (their uniform offset is 0 then, so
+    // that no range check can wrap around)
+    auto live = [&](int step) { return !ANY || z * steps + step < total; };
+    auto within = [&](const Span& s, int step) { return Span{s.base, live(step) ? s.bytes : 0u}; };
+    auto at = [&](uint32_t soff, int step) { return live(step) ? soff : 0u; };
 
     const int half = lane >> 5;
     // activations: rows of the tile past M read as zero
@@ -122,7 +137,8 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
     auto copy_x = [&](uint16_t* buf, int step) {
 #pragma unroll
         for (int c = 0; c < JT; ++c)
-            lds_copy16(xspan, buf + 512 * (JT * wave + c), xoff[c], 2 * (kbase + kStep * step));
+            lds_copy16(within(xspan, step), buf + 512 * (JT * wave + c), xoff[c],
+                       at(2 * (kbase + kStep * step), step));
     };
     const int swz = (lane & 7) ^ ((lane >> 3) & 1);
     uint32_t roff[4];
@@ -146,19 +162,35 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
                                             : (uint32_t)(32 * wave + (lane & 31));
     auto tile_row = [&](int r) { return (EPI == kWideSilu ? 64u : 128u) * r; };
     const uint32_t woff = wlane * rowb + (INT4 ? 16u : 32u) * half;
-    u32x4_t cw[W][R][CL];
+    u32x4_t cw[W][R][CW];
+    uint32_t cs[W][R], cz[W][R];  // SZ: the scale, the byte that holds the zero point
     u32x4_t ts[R], tsn[R];
     uint2 tz[R], tzn[R];
     uint32_t zsh = 0, zshn = 0;
-    auto load_w = [&](u32x4_t (&w)[R][CL], int step) {
+    // SZ: where this lane's zero point lies (group g of the row), and its nibble's shift
+    auto zero_at = [&](int step, uint32_t& sh) {
+        int zb;
+        zero_loc(min((kbase >> 5) + 2 * step + half, G - 1), G, zb, sh);
+        return (uint32_t)zb;
+    };
+    auto load_w = [&](int slot, int step) {
 #pragma unroll
-        for (int r = 0; r < R; ++r)
+        for (int r = 0; r < R; ++r) {
 #pragma unroll
-            for (int c = 0; c < CL; ++c)
-                w[r][c] = load16(wspan, woff + 16 * c, tile_row(r) * rowb + (INT4 ? kbase / 2 + 32 * step : kbase + 64 * step));
+            for (int c = 0; c < CW; ++c)
+                cw[slot][r][c] = load16(within(wspan, step), woff + 16 * c,
+                                        at(tile_row(r) * rowb + (INT4 ? kbase / 2 + 32 * step : kbase + 64 * step), step));
+            if constexpr (SZ) {
+                uint32_t sh;
+                cs[slot][r] = load_u16(within(sspan, step), wlane * (uint32_t)(2 * G) + 2 * half,
+                                       at(tile_row(r) * (uint32_t)(2 * G) + kbase / 16 + 4 * step, step));
+                cz[slot][r] = load_u8(within(zspan, step), wlane * (uint32_t)(G >> 1) + zero_at(step, sh),
+                                      at(tile_row(r) * (uint32_t)(G >> 1), step));
+            }
+        }
     };
     auto load_blk = [&](u32x4_t (&s)[R], uint2 (&zz)[R], uint32_t& sh, int blk) {
-        if constexpr (INT4) {
+        if constexpr (INT4 && !SZ) {
             int zb;
             zero_loc((kbase >> 5) + 8 * blk, G, zb, sh);
 #pragma unroll
@@ -185,7 +217,7 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
     for (int v = -kRing; v < 0; ++v) {
         if (v >= 1 - kRing) copy_x(ring[(v + kRing - 1) % 3], v + kRing - 1);
         cbar();
-        if (v + W >= 0) load_w(cw[v + W], v + W);
+        if (v + W >= 0) load_w(v + W, v + W);
         cbar();
     }
     MOSS_WAIT_VM(JT + 2 * R * CL);  // steps 0 and 1 have landed
@@ -194,9 +226,14 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
     const MixedUnpack mu = make_mixed_unpack();
 
     Group gd[R];
-    auto group = [&](auto ic, const u32x4_t (&s)[R], const uint2 (&zz)[R], uint32_t sh) {
+    auto group = [&](auto ic, const u32x4_t (&s)[R], const uint2 (&zz)[R], uint32_t sh, int step) {
         constexpr int i = decltype(ic)::value;
-        if constexpr (INT4) {
+        if constexpr (SZ) {
+            uint32_t lsh;
+            zero_at(step, lsh);
+#pragma unroll
+            for (int r = 0; r < R; ++r) gd[r] = make_group(cs[i % W][r], (cz[i % W][r] >> lsh) & 15u);
+        } else if constexpr (INT4) {
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 const uint32_t zw = i < 2 ? zz[r].x : zz[r].y;
@@ -205,7 +242,7 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
         }
     };
     // pair u of the A operand for word kk of this lane's group
-    auto pair = [&](auto uc, const u32x4_t (&w)[R][CL], int kk, int r) -> uint32_t {
+    auto pair = [&](auto uc, const u32x4_t (&w)[R][CW], int kk, int r) -> uint32_t {
         constexpr int u = decltype(uc)::value;
         if constexpr (INT4) return dequant_pair<u>(w[r][0][kk], mu.mask_hi, mu.f16_bias, gd[r]);
         else return fp8x2_to_bf16x2<u % 2 == 1>(w[r][kk >> 1][2 * (kk & 1) + u / 2]);
@@ -218,7 +255,7 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
     using Yes = std::true_type;
     u32x4_t a[R];
     bf16x8_t b[JT];
-    group(S0{}, ts, tz, zsh);
+    group(S0{}, ts, tz, zsh, 0);
 #pragma unroll
     for (int j = 0; j < JT; ++j) b[j] = read_b(X0, 0, j);
 #pragma unroll
@@ -238,7 +275,7 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
             constexpr bool more = !(LAST && i == kRing - 1 && kk == 3);  // another quarter follows
             constexpr int nk = (kk + 1) & 3;
             if constexpr (kk == 3 && more) {
-                if constexpr (INT4 && i == kRing - 1) {
+                if constexpr (INT4 && !SZ && i == kRing - 1) {
 #pragma unroll
                     for (int r = 0; r < R; ++r) {
                         ts[r] = tsn[r];
@@ -246,7 +283,7 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
                     }
                     zsh = zshn;
                 }
-                group(std::integral_constant<int, (i + 1) % kRing>{}, ts, tz, zsh);
+                group(std::integral_constant<int, (i + 1) % kRing>{}, ts, tz, zsh, s + 1);
             }
             const auto& w = cw[(kk == 3 ? i + 1 : i) % W];
             u32x4_t an[R];
@@ -275,8 +312,8 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
                 if (more) a[r] = an[r];
             if constexpr (kk == 2) {
                 // the step's codes have all been taken
-                if constexpr (codes) load_w(cw[i % W], s + W);
-                if constexpr (INT4 && !LAST && i == 0) load_blk(tsn, tzn, zshn, blk + 1);
+                if constexpr (codes) load_w(i % W, s + W);
+                if constexpr (INT4 && !SZ && !LAST && i == 0) load_blk(tsn, tzn, zshn, blk + 1);
                 cbar();
                 pin();
             }
@@ -366,6 +403,9 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
     }
     // C[n][m] of a 32 x 32 tile: lane l, element e -> n row 8 (e / 4) + 4 (l / 32) + e % 4, m column
     // l % 32; the four e of a quad are consecutive n (N % 4 == 0: a quad is all in range or all out)
+    const bool quads = !ANY || (N % 4 == 0 && (EPI == kWideSplit || reinterpret_cast<uintptr_t>(Y) % 8 == 0));
+    const bool pairs = N % 2 == 0 && (EPI == kWideSplit || reinterpret_cast<uintptr_t>(Y) % 4 == 0);
+    auto scaled = [&](float v, int n) { return !INT4 && row_scale ? v * row_scale[n] : v; };
 #pragma unroll
     for (int j = 0; j < JT; ++j) {
         const int m = m0 + 32 * j + (lane & 31);
@@ -378,7 +418,26 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
                 if (n >= N) continue;
                 const f32x16_t& c = acc[r][j];
                 const float v0 = c[4 * q], v1 = c[4 * q + 1], v2 = c[4 * q + 2], v3 = c[4 * q + 3];
-                if constexpr (EPI == kWideSplit) {
+                if (ANY && !quads) {  // outputs one by one, or in pairs for an even N
+                    const float v[4] = {v0, v1, v2, v3};
+#pragma unroll
+                    for (int e = 0; e < 4; e += 2) {
+                        const size_t o = (size_t)m * N + n + e;
+                        if (pairs && n + e < N) {
+                            if constexpr (EPI == kWideSplit)
+                                *reinterpret_cast<float2*>(part + (size_t)z * M * N + o) = make_float2(v[e], v[e + 1]);
+                            else
+                                *reinterpret_cast<uint32_t*>(Y + o) = pack_bf16x2(scaled(v[e], n + e), scaled(v[e + 1], n + e + 1));
+                        } else if (!pairs) {
+#pragma unroll
+                            for (int i = 0; i < 2; ++i) {
+                                if (n + e + i >= N) continue;
+                                if constexpr (EPI == kWideSplit) part[(size_t)z * M * N + o + i] = v[e + i];
+                                else Y[o + i] = f32_to_bf16(scaled(v[e + i], n + e + i));
+                            }
+                        }
+                    }
+                } else if constexpr (EPI == kWideSplit) {
                     *reinterpret_cast<float4*>(part + ((size_t)z * M + m) * N + n) = make_float4(v0, v1, v2, v3);
                 } else {
                     uint2 o;

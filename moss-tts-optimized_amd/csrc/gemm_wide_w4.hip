@@ -19,14 +19,25 @@ constexpr StepCost kStepCost[2][2] = {
     {{{330, 370, 400, 470, 560}, {275, 320, 385, 520, 555}}, {{0, 0, 740, 900, 1056}, {0, 0, 680, 880, 1100}}},
 };
 
+// Tiles of the any-shape form (one instance each costs what a regular one does; these lie within 15% of
+// the best regular tile at every size).
+constexpr bool any_tile(int r, int jt) { return r == 1 ? jt != 3 : jt == 4; }
+
 template <int R, int JT>
 int launch_tile(WideEpilogue epi, const WidePlan& p, const WideArgs& a, hipStream_t st) {
     const int bn = (epi == kWideSilu ? 64 : 128) * R;
     const dim3 grid((unsigned)(((a.M + 32 * JT - 1) / (32 * JT)) * ((a.N + bn - 1) / bn) * p.split));
-#define MOSS_WIDE(EPI)                                                                                               \
-    hipLaunchKernelGGL((gemm_wide_kernel<kInt4G32, R, JT, EPI>), grid, dim3(256), 0, st, (const uint16_t*)a.x,        \
+#define MOSS_WIDE(...)                                                                                               \
+    hipLaunchKernelGGL((gemm_wide_kernel<kInt4G32, R, JT, __VA_ARGS__>), grid, dim3(256), 0, st, (const uint16_t*)a.x,        \
                        (const uint8_t*)a.qw, (const uint16_t*)a.sc, (const uint8_t*)a.zp, a.row_scale, (uint16_t*)a.y, \
                        a.part, a.M, a.N, a.K, p.split, a.qr)
+    if constexpr (any_tile(R, JT)) {
+        if (p.any) {
+            if (epi == kWideSplit) MOSS_WIDE(kWideSplit, true);
+            else MOSS_WIDE(kWidePlain, true);
+            return moss_launch_status();
+        }
+    }
     if (epi == kWideSplit) MOSS_WIDE(kWideSplit);
     else if (epi == kWideSilu) MOSS_WIDE(kWideSilu);
     else if (epi == kWideQkRope) MOSS_WIDE(kWideQkRope);
@@ -40,8 +51,12 @@ int launch_tile(WideEpilogue epi, const WidePlan& p, const WideArgs& a, hipStrea
 // Whole blocks of four K steps and 4-output stores; INT4: the 8 zero bytes of every block on one
 // nibble side of their 128-group chunk (the last chunk a multiple of 16 groups long).  The weight lies
 // within the 32-bit offsets of the buffer instructions.
+bool wide_any_shape(int fmt, int K, int nw) {
+    return K % kStep == 0 && (long long)nw * K / (fmt == kInt4G32 ? 2 : 1) < 1ll << 31;
+}
+
 bool wide_shape(int fmt, int K, int nw) {
-    if (nw % 4 || K % (4 * kStep) || (long long)nw * K / (fmt == kInt4G32 ? 2 : 1) >= 1ll << 31) return false;
+    if (nw % 4 || K % (4 * kStep) || !wide_any_shape(fmt, K, nw)) return false;
     const int G = K / 32;
     return fmt == kFp8E4M3 || (G % 16 == 0 && (G % 128) % 16 == 0);
 }
@@ -49,31 +64,42 @@ bool wide_shape(int fmt, int K, int nw) {
 // The expected time of each tile and split is what the step costs above give for the workgroups per CU,
 // not less than the weights' bytes at 4.5 TB/s, and for a split the partial sums written and read back
 // (8 bytes each at 5 TB/s) and the launch that adds them.  A split leaves every workgroup at least two
-// blocks of K and its partials fit 32 MiB.
-WidePlan wide_plan(int fmt, int M, int K, int nw, int max_split) {
-    WidePlan best{1, 1, 1};
+// blocks of K and its partials fit 32 MiB.  The any-shape form, a few percent slower a step, is also
+// weighed where the regular one fits: it splits a K of any number of steps (e4m3 K = 6400 = 100 steps, M =
+// 10, N = 3000: 31.8 us whole, 9.8 split).
+static WidePlan plan(int fmt, int M, int K, int nw, int max_split, bool regular) {
+    WidePlan best{1, 1, 1, !regular};
     double least = 1e30;
     const double wbytes = (double)nw * K * (fmt == kInt4G32 ? 0.5625 : 1.0);
+    const int total = K / kStep;
     for (int r = 1; r <= 2; ++r)
         for (int jt = 1; jt <= 5; ++jt) {
             const StepCost& c = kStepCost[fmt][r - 1];
             if (!c.alone[jt - 1] || (jt > 1 && 32 * (jt - 1) >= M)) continue;
             const long tiles = (long)((M + 32 * jt - 1) / (32 * jt)) * ((nw + 128 * r - 1) / (128 * r));
             for (int split = 1; split <= max_split; split *= 2) {
-                const int steps = K / kStep / split;
-                if (split > 1 && (K / kStep % (4 * split) || steps < 8 || (long long)split * M * nw * 4 > 32ll << 20)) break;
+                const bool any = !regular || total % (4 * split);  // the regular form: whole blocks of four steps
+                if (any && !any_tile(r, jt)) break;
+                const int steps = any ? ((total + split - 1) / split + 3) & ~3 : total / split;
+                if (split > 1 && (steps < 8 || (long long)split * M * nw * 4 > 32ll << 20)) break;
                 const long per_cu = (tiles * split + 255) / 256;
-                const double ns = per_cu == 1 ? c.alone[jt - 1] : (double)per_cu * c.shared[jt - 1];
+                const double ns = (any ? 1.06 : 1.0) * (per_cu == 1 ? c.alone[jt - 1] : (double)per_cu * c.shared[jt - 1]);
                 double us = 3.5 + std::max(steps * ns / 1000, wbytes / 4.5e6);
                 if (split > 1) us += 2.5 + (double)split * M * nw * 8 / 5e6;
                 if (us < least) {
                     least = us;
-                    best = {r, jt, split};
+                    best = {r, jt, split, any};
                 }
             }
         }
     return best;
 }
+
+WidePlan wide_plan(int fmt, int M, int K, int nw, int max_split) {
+    return plan(fmt, M, K, nw, max_split, wide_shape(fmt, K, nw));
+}
+
+WidePlan wide_plan_any(int fmt, int M, int K, int nw, int max_split) { return plan(fmt, M, K, nw, max_split, false); }
 
 int wide_launch_w4(WideEpilogue epi, const WidePlan& p, const WideArgs& a, hipStream_t st) {
     switch (10 * p.r + p.jt) {

@@ -656,6 +656,25 @@ __global__ __launch_bounds__(256) void gemm_reduce(const float* __restrict__ par
     *reinterpret_cast<uint2*>(Y + i) = o;
 }
 
+// The same, one output per thread, for any N.
+__global__ __launch_bounds__(256) void gemm_reduce_any(const float* __restrict__ part,
+                                                       const float* __restrict__ row_scale, uint16_t* __restrict__ Y,
+                                                       int MN, int N, int S) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= MN) return;
+    float acc = 0.f;
+    for (int z0 = 0; z0 < S; z0 += 4) {
+        float v[4];
+#pragma unroll
+        for (int z = 0; z < 4; ++z)
+            if (z0 + z < S) v[z] = part[(size_t)(z0 + z) * MN + i];
+#pragma unroll
+        for (int z = 0; z < 4; ++z)
+            if (z0 + z < S) acc += v[z];
+    }
+    Y[i] = f32_to_bf16(row_scale ? acc * row_scale[i % N] : acc);
+}
+
 // The same over [M, 2 N] gate||up sums followed by the SiLU*mul: Y[m, n] = bf16(bf16(silu(g)) u) of the
 // bf16-rounded sums g = [m, n], u = [m, N + n], bit for bit what gemm_reduce and moss_silu_mul give.
 __global__ __launch_bounds__(256) void gemm_reduce_silu(const float* __restrict__ part, uint16_t* __restrict__ Y,
@@ -922,7 +941,7 @@ Plan plan_gemm(int M, int K, int N, bool int4) {
 }
 
 int wide_max_split(int fmt, int M, int K, int N) {
-    return fmt == kInt4G32 && M > 64 && plan_gemm(M, K, N, true).split == 1 ? 1 : 16;
+    return fmt == kInt4G32 && M > 64 && reg_tile_shape(K, N, true) && plan_gemm(M, K, N, true).split == 1 ? 1 : 16;
 }
 
 Plan plan_lds(int M, int K, int N) {
@@ -990,12 +1009,17 @@ bool tokens_gemv(int M, int K, const void* x, const void* qw) {
 
 void reduce_parts(const void* part, const float* row_scale, void* y, int M, int N, int split, hipStream_t st) {
     const int mn = M * N;
+    if (N % 4 || !MOSS_ALIGNED(y, 8)) {
+        hipLaunchKernelGGL(gemm_reduce_any, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, st, (const float*)part,
+                           row_scale, (uint16_t*)y, mn, N, split);
+        return;
+    }
     hipLaunchKernelGGL(gemm_reduce, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, st, (const float*)part,
                        row_scale, (uint16_t*)y, mn, N, split);
 }
 
 bool split_fits(int split, const void* ws, long long ws_bytes, const void* y, int M, int N) {
-    return split == 1 || (ws && ws_bytes >= (long long)split * M * N * 4 && MOSS_ALIGNED(ws, 16) && MOSS_ALIGNED(y, 8));
+    return split == 1 || (ws && ws_bytes >= (long long)split * M * N * 4 && MOSS_ALIGNED(ws, 16));
 }
 
 // Where the weight-streaming kernel, which never splits K over workgroups, still beats the wide tile with
@@ -1010,19 +1034,26 @@ bool stream_better(int fmt, int M, int K, int N) {
     return fmt == kFp8E4M3 && mk <= (N >= 16384 ? 12 : 5) * 4096;
 }
 
-// Whether the wide tile (gemm_wide_kernel.h) takes a call, and how.  Above 64 INT4 tokens it splits K
+// Whether the wide tile (gemm_wide_kernel.h) takes a call, and how.  Shapes without whole blocks of K or
+// quads of N and misaligned pointers take its any-shape form (INT4 M = 150, K = 4160, N = 1001: 36.9 -> 18.0 us
+// against the LDS tiles, M = 600, K = 11008, N = 4100: 158 -> 111).  Above 64 INT4 tokens it splits K
 // only where plan_gemm does: there the fused epilogues run without a workspace, and the plain GEMM
 // of the same shape sums in the same order.  A call whose planned split finds no workspace goes to the
 // weight-streaming kernel if that takes it (K = N = 4096, M = 24: 10 us against 24 us unsplit).
 bool choose_wide(int fmt, int M, int K, int N, const void* x, const void* qw, const void* sc, const void* zp,
                  const void* y, const void* ws, long long ws_bytes, WidePlan& p) {
-    if (!wide_shape(fmt, K, N) || !MOSS_ALIGNED(y, 8)) return false;
-    if (fmt == kInt4G32 && !(MOSS_ALIGNED(sc, 16) && MOSS_ALIGNED(zp, 8))) return false;
-    if (stream_shape(fmt, M, K, N, x, qw, sc, zp, y) && stream_better(fmt, M, K, N)) return false;
-    p = wide_plan(fmt, M, K, N, wide_max_split(fmt, M, K, N));
+    const bool aligned = MOSS_ALIGNED(y, 8) && (fmt == kFp8E4M3 || (MOSS_ALIGNED(sc, 16) && MOSS_ALIGNED(zp, 8)));
+    const bool any = !(wide_shape(fmt, K, N) && aligned);
+    if (any && !(wide_any_shape(fmt, K, N) && MOSS_ALIGNED(sc, 2))) return false;
+    const bool stream = stream_shape(fmt, M, K, N, x, qw, sc, zp, y);
+    if (stream && stream_better(fmt, M, K, N)) return false;
+    auto plan = [&](int max_split) {
+        return any ? wide_plan_any(fmt, M, K, N, max_split) : wide_plan(fmt, M, K, N, max_split);
+    };
+    p = plan(wide_max_split(fmt, M, K, N));
     if (split_fits(p.split, ws, ws_bytes, y, M, N)) return true;
-    if (stream_shape(fmt, M, K, N, x, qw, sc, zp, y)) return false;
-    p = wide_plan(fmt, M, K, N, 1);
+    if (stream) return false;
+    p = plan(1);
     return true;
 }
 
@@ -1106,7 +1137,7 @@ long long gemm_workspace_bytes(int M, int K, int N) {
     for (const Plan& p : {plan_gemm(M, K, N, true), plan_gemm(M, K, N, false), plan_lds(M, K, N)})
         if (p.split > 1) bytes = std::max(bytes, (long long)p.split * M * N * 4);
     for (int fmt : {(int)kInt4G32, (int)kFp8E4M3})
-        if (wide_shape(fmt, K, N)) {
+        if (wide_any_shape(fmt, K, N)) {
             const int split = wide_plan(fmt, M, K, N, wide_max_split(fmt, M, K, N)).split;
             if (split > 1) bytes = std::max(bytes, (long long)split * M * N * 4);
         }
@@ -1161,7 +1192,7 @@ MOSS_API int moss_w4g32_gemm_silu(const void* x, const void* qw, const void* sc,
     char* ws = (char*)workspace;
     WidePlan wp;
     if (!tokens_gemv(M, K, x, qw) && MOSS_ALIGNED(y, 8) &&
-        choose_wide(kInt4G32, M, K, 2 * N, x, qw, sc, zp, ws, ws + inter, workspace_bytes - inter, wp) && wp.split == 1)
+        choose_wide(kInt4G32, M, K, 2 * N, x, qw, sc, zp, ws, ws + inter, workspace_bytes - inter, wp) && wp.split == 1 && !wp.any)
         return wide_launch_w4(kWideSilu, wp, WideArgs{x, qw, sc, zp, nullptr, y, nullptr, M, K, N, QkRope{}}, st);
     int split = 1;
     if (int rc = launch_gemm<kInt4G32>(x, qw, sc, zp, ws, M, K, 2 * N, nullptr, ws + inter, workspace_bytes - inter, st,

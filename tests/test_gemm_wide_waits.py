@@ -86,7 +86,7 @@ def test_check_rejects_a_lax_wait():
         check_ring_waits(body, 1)
 
 
-@pytest.mark.parametrize("source,instances", [("gemm_wide_w4.hip", 28), ("gemm_wide_fp8.hip", 16)])
+@pytest.mark.parametrize("source,instances", [("gemm_wide_w4.hip", 38), ("gemm_wide_fp8.hip", 26)])
 def test_ring_waits_cover_every_copy(tmp_path, source, instances):
     bodies = _bodies(source, tmp_path)
     assert len(bodies) == instances

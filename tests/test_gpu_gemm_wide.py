@@ -26,9 +26,11 @@ def _close(y, ref):
 SHAPES = [(1, 512, 128), (31, 512, 132), (33, 1024, 260), (65, 512, 516), (96, 4096, 1028), (97, 4096, 2052),
           (129, 4096, 4096), (161, 12288, 2052), (320, 4096, 6144), (301, 4608, 4100), (1000, 1024, 8200),
           (513, 4096, 12292), (6, 12288, 4096)]
+# the any-shape form: K of one step to many with and without a rest, any N, a K split with a rest
+ANY = [(5, 64, 5), (33, 192, 130), (16, 320, 64), (65, 4160, 1001), (150, 4032, 515), (301, 12224, 258), (700, 1088, 4099)]
 
 
-@pytest.mark.parametrize("m,k,n", SHAPES)
+@pytest.mark.parametrize("m,k,n", SHAPES + ANY)
 def test_int4_matches_float32(dev, m, k, n):
     from moss_tts._runtime import w4g32
 
@@ -38,7 +40,7 @@ def test_int4_matches_float32(dev, m, k, n):
     _close(w4g32.gemm(x, pw), x.float() @ w4g32.dequantize(pw).float().T)
 
 
-@pytest.mark.parametrize("m,k,n", [(2, 256, 132)] + SHAPES[1:])
+@pytest.mark.parametrize("m,k,n", [(2, 256, 132)] + SHAPES[1:] + ANY)
 def test_fp8_matches_float32(dev, m, k, n):
     from moss_tts._runtime import fp8
 
