@@ -1045,6 +1045,9 @@ bool choose_wide(int fmt, int M, int K, int N, const void* x, const void* qw, co
     const bool aligned = MOSS_ALIGNED(y, 8) && (fmt == kFp8E4M3 || (MOSS_ALIGNED(sc, 16) && MOSS_ALIGNED(zp, 8)));
     const bool any = !(wide_shape(fmt, K, N) && aligned);
     if (any && !(wide_any_shape(fmt, K, N) && MOSS_ALIGNED(sc, 2))) return false;
+    // a K of a few steps at 33 .. 64 tokens and N % 4 != 0 stays in the 64-token LDS tiles (M = 50, K = 320, N =
+    // 3001: 5.1 against 6.2 us; M = 40, K = 704, N = 16383: 7.7 / 8.7; K = 768: equal; M = 72, K = 256: 6.0 / 4.6)
+    if (any && fmt == kInt4G32 && N % 4 && M > 32 && M <= 64 && K < 768) return false;
     const bool stream = stream_shape(fmt, M, K, N, x, qw, sc, zp, y);
     if (stream && stream_better(fmt, M, K, N)) return false;
     auto plan = [&](int max_split) {
