@@ -7,10 +7,12 @@ namespace moss {
 namespace {
 
 // Nanoseconds a workgroup takes per K step of 64, by tile (columns JT = 1 .. 5): `alone`, with a CU to
-// itself, and `shared`, per workgroup with two on the CU.  Medians over M = 5 .. 2048 on the four
-// projections of the 4096 / 12288 model (K 4096 and 12288, N 4096 .. 24576), within 10% of nearly all
-// of them; 0: no such instance (R = 2 below 3 token tiles lost to R = 1 everywhere, and INT4 at 2 x 5
-// spills).
+// itself, and `shared`, per workgroup with two on the CU.  From timings of every tile and split at 45
+// shapes (M = 5 .. 2048 on the four projections of the 4096 / 12288 model), taken where most CUs have work:
+// fewer busy CUs hold a higher clock and a step takes down to 0.75 of this.  By these costs the chosen
+// tile and split, with the partial sums' cost, was the best measured one at 34 of the 45 shapes, within 6%
+// of it at 39 and within 14% at all.  0: no such instance (R = 2 below 3 token tiles was nowhere the best,
+// and INT4 at 2 x 5 spills).
 struct StepCost {
     int alone[5], shared[5];
 };
@@ -19,8 +21,7 @@ constexpr StepCost kStepCost[2][2] = {
     {{{330, 370, 400, 470, 560}, {275, 320, 385, 520, 555}}, {{0, 0, 740, 900, 1056}, {0, 0, 680, 880, 1100}}},
 };
 
-// Tiles of the any-shape form (one instance each costs what a regular one does; these lie within 15% of
-// the best regular tile at every size).
+// Tiles of the any-shape form: a subset, to keep the library small.
 constexpr bool any_tile(int r, int jt) { return r == 1 ? jt != 3 : jt == 4; }
 
 template <int R, int JT>
