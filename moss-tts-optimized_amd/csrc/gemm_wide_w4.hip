@@ -11,7 +11,7 @@ namespace {
 // shapes (M = 5 .. 2048 on the four projections of the 4096 / 12288 model), taken where most CUs have work:
 // fewer busy CUs hold a higher clock and a step takes down to 0.75 of this.  By these costs the chosen
 // tile and split, with the partial sums' cost, was the best measured one at 34 of the 45 shapes, within 6%
-// of it at 39 and within 14% at all.  0: no such instance (R = 2 below 3 token tiles was nowhere the best,
+// of it at 41 and within 17% at all.  0: no such instance (R = 2 below 3 token tiles was nowhere the best,
 // and INT4 at 2 x 5 spills).
 struct StepCost {
     int alone[5], shared[5];
@@ -64,10 +64,10 @@ bool wide_shape(int fmt, int K, int nw) {
 
 // The expected time of each tile and split is what the step costs above give for the workgroups per CU,
 // not less than the weights' bytes at 4.5 TB/s, and for a split the partial sums written and read back
-// (8 bytes each at 5 TB/s) and the launch that adds them.  A split leaves every workgroup at least two
-// blocks of K and its partials fit 32 MiB.  The any-shape form, a few percent slower a step, is also
+// (8 bytes each at 8 TB/s: they mostly stay in the last-level cache) and the launch that adds them, 6 us for
+// two of 512 x 4096.  A split leaves every workgroup at least two blocks of K and its partials fit 32 MiB.  The any-shape form, a few percent slower a step, is also
 // weighed where the regular one fits: it splits a K of any number of steps (e4m3 K = 6400 = 100 steps, M =
-// 10, N = 3000: 31.8 us whole, 9.8 split).
+// 10, N = 3000: 31.8 us whole, 11.4 split).
 static WidePlan plan(int fmt, int M, int K, int nw, int max_split, bool regular) {
     WidePlan best{1, 1, 1, !regular};
     double least = 1e30;
@@ -86,7 +86,7 @@ static WidePlan plan(int fmt, int M, int K, int nw, int max_split, bool regular)
                 const long per_cu = (tiles * split + 255) / 256;
                 const double ns = (any ? 1.06 : 1.0) * (per_cu == 1 ? c.alone[jt - 1] : (double)per_cu * c.shared[jt - 1]);
                 double us = 3.5 + std::max(steps * ns / 1000, wbytes / 4.5e6);
-                if (split > 1) us += 2.5 + (double)split * M * nw * 8 / 5e6;
+                if (split > 1) us += 2.0 + (double)split * M * nw * 8 / 8e6;
                 if (us < least) {
                     least = us;
                     best = {r, jt, split, any};
