@@ -413,11 +413,14 @@ MOSS_API int moss_embedding_sum(const void* ids, const void* text, const void* a
                                 int Vt, int V, int Q, void* stream) {
     MOSS_CHECK_ARG(ids && text && audio && out && T > 0 && H > 0 && Vt > 0 && V > 0 && Q >= 0);
     // 16- or 8-byte loads where rows allow them: 512 tokens x 33 rows of 4096 in 50 us with 2-byte loads
-    if (H % 8 == 0 && MOSS_ALIGNED(text, 16) && MOSS_ALIGNED(audio, 16) && MOSS_ALIGNED(out, 16))
+    // -- and one value per thread for a few tokens, whose time is the chain of 33 rounded additions per value
+    // and not the loads (one token: the decode step 237.5 -> 235.7 us, its W4A8 form 221.8 -> 219.0)
+    const bool few = (long long)T * H <= 4 * 4096;
+    if (!few && H % 8 == 0 && MOSS_ALIGNED(text, 16) && MOSS_ALIGNED(audio, 16) && MOSS_ALIGNED(out, 16))
         hipLaunchKernelGGL(embedding_sum_rows<8>, dim3(T, (H / 8 + 255) / 256), dim3(256), 0, (hipStream_t)stream,
                            (const int64_t*)ids, (const uint16_t*)text, (const uint16_t*)audio, (uint16_t*)out, H, Vt,
                            V, Q);
-    else if (H % 4 == 0 && MOSS_ALIGNED(text, 8) && MOSS_ALIGNED(audio, 8) && MOSS_ALIGNED(out, 8))
+    else if (!few && H % 4 == 0 && MOSS_ALIGNED(text, 8) && MOSS_ALIGNED(audio, 8) && MOSS_ALIGNED(out, 8))
         hipLaunchKernelGGL(embedding_sum_rows<4>, dim3(T, (H / 4 + 255) / 256), dim3(256), 0, (hipStream_t)stream,
                            (const int64_t*)ids, (const uint16_t*)text, (const uint16_t*)audio, (uint16_t*)out, H, Vt,
                            V, Q);
