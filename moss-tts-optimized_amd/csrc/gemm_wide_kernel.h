@@ -160,7 +160,12 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
     const Span zspan{zp + (INT4 ? (size_t)n0 * (G >> 1) : 0), rows * (uint32_t)(G >> 1)};
     const uint32_t wlane = EPI == kWideSilu ? (uint32_t)(16 * wave + (lane & 15) + ((lane >> 4) & 1) * N)
                                             : (uint32_t)(32 * wave + (lane & 31));
-    auto tile_row = [&](int r) { return (EPI == kWideSilu ? 64u : 128u) * r; };
+    // A row tile that starts past the last row reads tile 0's rows again and stores none of them: a uniform
+    // offset at or past the end of a span would wrap the range check (offset >= bytes - uniform offset).
+    auto tile_row = [&](int r) {
+        const uint32_t row = (EPI == kWideSilu ? 64u : 128u) * r;
+        return row < rows ? row : 0u;
+    };
     const uint32_t woff = wlane * rowb + (INT4 ? 16u : 32u) * half;
     u32x4_t cw[W][R][CW];
     uint32_t cs[W][R], cz[W][R];  // SZ: the scale, the byte that holds the zero point

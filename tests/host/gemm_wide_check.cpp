@@ -1,0 +1,104 @@
+// Host checks of the wide GEMM tile, compiled against hip_on_host.h.
+//   bounds          every instance, over remainders of M, N and K: addresses of every read, and stores
+//   plan            reads "format M K N" lines, prints what the dispatch picks for each
+#include "w4g32_gemm.hip"
+
+namespace moss {
+int qk_rope_from_parts(const float*, int, const void*, const void*, const void*, const void*, void*, void*, void*,
+                       const void*, int, int, float, hipStream_t) { return 0; }
+int addnorm_from_parts(const float*, int, const void*, const void*, void*, void*, int, int, float, hipStream_t) { return 0; }
+int add_rmsnorm_inplace(void*, const void*, const void*, void*, int, int, float, hipStream_t) { return 0; }
+bool w4g32_gemv_tokens_shape(int M, int K) { return M >= 2 && M <= 4 && K <= 16384; }
+int w4g32_gemv_tokens_launch(const void*, const void*, const void*, const void*, void*, int, int, int, hipStream_t) { return 0; }
+}  // namespace moss
+extern "C" int moss_silu_mul(const void*, void*, int, int, void*) { return 0; }
+extern "C" int moss_rmsnorm(const void*, const void*, const void*, void*, void*, int, int, float, void*) { return 0; }
+extern "C" int moss_qk_norm_rope_kv(const void*, const void*, const void*, const void*, const void*, void*, void*, void*,
+                                    const void*, int, int, float, int, void*) { return 0; }
+
+// An array whose neighbours on both sides are watched.
+template <class T>
+struct Watched {
+    static constexpr size_t kGuard = 4096;
+    std::vector<T> all;
+    size_t n;
+    Watched(size_t n_) : all(n_ + 2 * kGuard, (T)77), n(n_) {}
+    T* data() { return all.data() + kGuard; }
+    bool intact() const {
+        for (size_t i = 0; i < kGuard; ++i)
+            if (all[i] != (T)77 || all[kGuard + n + i] != (T)77) return false;
+        return true;
+    }
+};
+
+static std::vector<char> operand(size_t bytes) {
+    std::vector<char> v(std::max<size_t>(bytes, 1));
+    operands.push_back({v.data(), bytes});
+    return v;
+}
+
+static int runs;
+static bool check(int fmt, WidePlan p, WideEpilogue epi, int M, int N, int K) {
+    const int nw = epi == kWideSilu ? 2 * N : N, G = K / 32, L = 64, before = (int)violations;
+    const bool int4 = fmt == kInt4G32;
+    operands.clear();
+    std::vector<char> x = operand((size_t)M * K * 2), qw = operand((size_t)nw * K / (int4 ? 2 : 1)),
+                      sc = operand(int4 ? (size_t)nw * G * 2 : 0), zp = operand(int4 ? (size_t)nw * G / 2 : 0);
+    Watched<uint16_t> y((size_t)M * (epi == kWideQkRope ? 4096 : N)), kc(8 * L * 128), vc(8 * L * 128);
+    Watched<float> part(epi == kWideSplit ? (size_t)p.split * M * N : 1);
+    std::vector<float> scale(int4 ? 1 : N);
+    std::vector<uint16_t> row(128), table(L * 128);
+    std::vector<int64_t> pos(M, L - 1);
+    const QkRope qr{row.data(), row.data(), table.data(), table.data(), kc.data(), vc.data(), pos.data(), L, 1e-6f};
+    const WideArgs a{x.data(), qw.data(), sc.data(), zp.data(), int4 ? nullptr : scale.data(), y.data(), part.data(), M, K, N, qr};
+    const int rc = int4 ? wide_launch_w4(epi, p, a, nullptr) : wide_launch_fp8(epi, p, a, nullptr);
+    ++runs;
+    const bool ok = rc == 0 && violations == before && y.intact() && part.intact() && kc.intact() && vc.intact();
+    if (!ok)
+        printf("FAIL format %d tile %d x %d any %d split %d epilogue %d M %d N %d K %d: rc %d\n", fmt, p.r, p.jt, p.any,
+               p.split, epi, M, N, K, rc);
+    return ok;
+}
+
+static bool bounds() {
+    static const int tiles[][2] = {{1, 1}, {1, 2}, {1, 3}, {1, 4}, {1, 5}, {2, 3}, {2, 4}, {2, 5}};
+    bool ok = true;
+    for (int fmt : {(int)kInt4G32, (int)kFp8E4M3})
+        for (auto& t : tiles) {
+            const int r = t[0], jt = t[1], bn = 128 * r;
+            if (fmt == kInt4G32 && r == 2 && jt == 5) continue;
+            // one row past a tile, rows that end in its first and in its second row tile, one short of it
+            for (int n : {4, 124, 128, 132, 252, 256, bn + 4, bn + 128, bn + 132, 2 * bn - 4}) {
+                const int m = 32 * jt + 1;
+                ok &= check(fmt, {r, jt, 1, false}, kWidePlain, m, n, 512);
+                ok &= check(fmt, {r, jt, 2, false}, kWideSplit, m, n, 512);
+                if (fmt == kInt4G32) ok &= check(fmt, {r, jt, 1, false}, kWideSilu, m, n, 512);
+            }
+            if (fmt == kInt4G32) ok &= check(fmt, {r, jt, 1, false}, kWideQkRope, 32 * jt - 1, 6144, 512);
+            if (r == 1 ? jt == 3 : jt != 4) continue;  // no any-shape instance
+            for (int n : {1, 127, 128, 129, 255, bn + 1, bn + 128, 2 * bn - 1})
+                for (int k : {64, 576}) {
+                    ok &= check(fmt, {r, jt, 1, true}, kWidePlain, 32 * jt - 1, n, k);
+                    // shares of K past its end among them
+                    for (int split : {2, 4}) ok &= check(fmt, {r, jt, split, true}, kWideSplit, 33, n, k);
+                }
+        }
+    printf("%d launches\n", runs);
+    return ok;
+}
+
+int main(int argc, char** argv) {
+    if (argc > 1 && !strcmp(argv[1], "bounds")) return bounds() ? 0 : 1;
+    run_launches = false;
+    int fmt, M, K, N;
+    const void* p = (const void*)4096;  // aligned for everything, never read
+    while (scanf("%d %d %d %d", &fmt, &M, &K, &N) == 4) {
+        WidePlan w{0, 0, 0, false};
+        const long long ws = gemm_workspace_bytes(M, K, N);
+        if (!(fmt == kInt4G32 && tokens_gemv(M, K, p, p))) {
+            if (!choose_wide(fmt, M, K, N, p, p, p, p, p, p, ws, w)) w = WidePlan{0, 0, 0, false};
+        }
+        printf("%d %d %d %d %lld\n", w.r, w.jt, w.split, (int)w.any, ws);
+    }
+    return 0;
+}

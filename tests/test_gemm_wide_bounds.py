@@ -1,0 +1,42 @@
+"""The wide GEMM tile (csrc/gemm_wide_kernel.h) compiled for the host against tests/host/hip_on_host.h:
+every lane of every workgroup runs on the CPU, and each buffer read is held against the documented range
+rule (lane offset below num_records - uniform offset, unsigned) and against the operand it belongs to.
+The values that rows past the weight give are never stored, so no output shows a read out of range."""
+import os
+import re
+import subprocess
+
+import pytest
+
+from moss_tts import _build
+
+HOST = os.path.join(os.path.dirname(os.path.abspath(__file__)), "host")
+_ASM = re.compile(r"\basm( volatile)?\((?:[^()]|\([^()]*\))*\);")  # device instructions, none with an address
+_SOURCES = ("common.h", "gemm_wide.h", "gemm_wide_kernel.h", "gemm_wide_w4.hip", "gemm_wide_fp8.hip", "w4g32_gemm.hip")
+
+
+@pytest.fixture(scope="session")
+def gemm_wide_check(tmp_path_factory):
+    clang = "/opt/rocm/llvm/bin/clang++"
+    if not os.path.exists(clang):
+        pytest.skip("clang++ not available")
+    d = tmp_path_factory.mktemp("gemm_wide")
+    (d / "hip").mkdir()
+    (d / "hip" / "hip_runtime.h").write_text(f'#include "{HOST}/hip_on_host.h"\n')
+    for name in _SOURCES:
+        with open(os.path.join(_build.CSRC, name)) as f:
+            (d / name).write_text(_ASM.sub(";", f.read()))
+    units = ["gemm_wide_w4.hip", "gemm_wide_fp8.hip", os.path.join(HOST, "gemm_wide_check.cpp")]
+    jobs = [subprocess.Popen([clang, "-std=c++17", "-O1", "-w", "-x", "c++", "-I", str(d), "-c", u, "-o", f"{i}.o"], cwd=d,
+                             stderr=subprocess.PIPE, text=True) for i, u in enumerate(units)]
+    for job in jobs:
+        err = job.communicate()[1]
+        assert job.returncode == 0, err[-3000:]
+    subprocess.run([clang, "0.o", "1.o", "2.o", "-o", "check"], cwd=d, check=True)
+    return str(d / "check")
+
+
+def test_reads_and_stores_stay_in_bounds(gemm_wide_check):
+    r = subprocess.run([gemm_wide_check, "bounds"], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout[-3000:]
+    assert "launches" in r.stdout
