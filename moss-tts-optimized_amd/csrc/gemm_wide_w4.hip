@@ -49,13 +49,14 @@ int launch_tile(WideEpilogue epi, const WidePlan& p, const WideArgs& a, hipStrea
 
 }  // namespace
 
-// Whole blocks of four K steps and 4-output stores; INT4: the 8 zero bytes of every block on one
-// nibble side of their 128-group chunk (the last chunk a multiple of 16 groups long).  The weight lies
-// within the 32-bit offsets of the buffer instructions.
+// The weight, and the activations of the deepest tile (160 rows of 2 K bytes), lie within the 32-bit offsets
+// of the buffer instructions.
 bool wide_any_shape(int fmt, int K, int nw) {
-    return K % kStep == 0 && (long long)nw * K / (fmt == kInt4G32 ? 2 : 1) < 1ll << 31;
+    return K % kStep == 0 && (long long)nw * K / (fmt == kInt4G32 ? 2 : 1) < 1ll << 31 && 320ll * K < 1ll << 32;
 }
 
+// Whole blocks of four K steps and 4-output stores; INT4: the 8 zero bytes of every block on one
+// nibble side of their 128-group chunk (the last chunk a multiple of 16 groups long).
 bool wide_shape(int fmt, int K, int nw) {
     if (nw % 4 || K % (4 * kStep) || !wide_any_shape(fmt, K, nw)) return false;
     const int G = K / 32;

@@ -40,3 +40,19 @@ def test_reads_and_stores_stay_in_bounds(gemm_wide_check):
     r = subprocess.run([gemm_wide_check, "bounds"], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout[-3000:]
     assert "launches" in r.stdout
+
+
+def _plans(check, calls):
+    """(r, jt, split, any, workspace bytes) of each (format, M, K, N) call with aligned operands; r = 0: not the
+    wide tile."""
+    text = "\n".join(" ".join(map(str, c)) for c in calls)
+    r = subprocess.run([check, "plan"], input=text, capture_output=True, text=True, check=True)
+    return [tuple(map(int, line.split())) for line in r.stdout.splitlines()]
+
+
+def test_offsets_fit_32_bits(gemm_wide_check):
+    # activations: 160 rows of 2 K bytes; weights: 2 GiB
+    last = (2 ** 32 // 320) // 256 * 256
+    calls = [(f, 160, k, 4) for f in (0, 1) for k in (last, last + 256, 2 ** 24)]
+    calls += [(0, 160, 4096, 2 ** 20 - 4), (0, 160, 4096, 2 ** 20), (1, 160, 4096, 2 ** 19 - 4), (1, 160, 4096, 2 ** 19)]
+    assert [p[0] > 0 for p in _plans(gemm_wide_check, calls)] == [True, False, False] * 2 + [True, False] * 2
