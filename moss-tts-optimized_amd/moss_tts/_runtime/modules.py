@@ -44,9 +44,10 @@ class QuantLinearG32(nn.Module):
         _require(weight.is_cuda and weight.ndim == 2, "a 2-D device weight [out, in] is required")
         w = weight.detach().float().contiguous()
         packed, check = w4g32.quantize_launch(w, symmetric)
-        module = cls(packed, **kw)
-        check()  # after the module is made: the device quantizes meanwhile
-        return module
+        try:
+            return cls(packed, **kw)  # made while the device quantizes
+        finally:
+            check()  # also where making it raises: the kernel may write the host flag until then
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if not (x.shape[-1] == self.in_features):

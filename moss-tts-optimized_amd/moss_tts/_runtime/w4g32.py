@@ -168,7 +168,8 @@ def import_signed(packed: torch.Tensor, scales: torch.Tensor) -> PackedW4G32:
 
 def quantize_launch(w: torch.Tensor, symmetric: bool):
     """Launches a quantizer; returns the weight and the check to call before using it, which waits for the
-    stream and raises unless every scale is in range.  The kernel sets a host flag where a scale is formed."""
+    stream and raises unless every scale is in range.  The kernel sets a flag in host memory where a scale is
+    formed, and that memory lives as long as the check: the caller calls it on every path, its own errors too."""
     _cuda_contig("w", w, torch.float32)
     _require(w.ndim == 2 and w.shape[1] % 64 == 0, "w must be [N, K] with K % 64 == 0")
     _require(_aligned(w, 16), "w must be 16-byte aligned")
