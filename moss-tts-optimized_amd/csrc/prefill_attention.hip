@@ -10,17 +10,21 @@
 //
 // Tiling (flash-attention style, online softmax in fp32): one workgroup per (32-token query tile,
 // HPW query heads of one KV head), KS waves per head: wave (kq, hw) takes query head hw of the group
-// and part kq of every block of 32 SUB KS keys, so a block's keys are split over the KS waves
-// of a head and the serial chain of blocks is KS times shorter than one wave per head would make
-// it.  Shapes: 2 heads x 4 parts of 32 keys while 16 workgroups per 32 tokens fill at most
-// one per CU, else 4 heads x 2 parts of 64 keys.  Tiles are issued longest first.
+// and the 32-key tiles kq, kq + KS, .. (SUB of them) of every block of 32 SUB KS keys, so a block's keys are
+// split over the KS waves of a head and the serial chain of blocks is KS times shorter than one wave per head
+// would make it.  Shapes: 2 heads x 4 waves of one tile while 16 workgroups per 32 tokens fill at most
+// one per CU, else 4 heads x 2 waves of two tiles.  Query tiles are issued longest first.
 // What bounds it: the vector work and the serial chain of a block (two waves a SIMD, S before the
-// softmax before P V).  Per 32 keys and wave that was about 220 VALU instructions to 16 MFMAs; now about 130:
-// the running reference of the softmax moves, and O^T is rescaled, only when a score passes it by 2^8;
-// the scale goes into the exponent's fma; masked blocks are a branch of their own; and rows past the
-// last visible key are zeros of the buffer reads, not branches around loads.  Two 32-key tiles a wave and
-// block halve the barriers and give S two independent MFMA chains.  2048 tokens: 117 -> 82 us (416 TFLOP/s),
-// 1024: 34.7 -> 26.0, 512: 14.7 -> 13.1, 150 after 600: 17.3 -> 15.2.
+// softmax before P V).  Against 32-key parts with a test around every load and a mask on every block: masked
+// blocks are a branch of their own, rows past the last visible key are zeros of the buffer reads, and two tiles a
+// wave and block halve the barriers and give S two independent MFMA chains.  2048 tokens: 110 -> 91 us
+// (377 TFLOP/s), 1024: 32.0 -> 27.2, 512: 12.8 -> 11.8, 150 after 600: 16.0 -> 14.7; the outputs are the same bit
+// for bit, since a wave's tiles, their order and the arithmetic of each are.
+// Precision: P is rounded to bf16 for the matrix cores, so a query's reference is its largest score so far,
+// tile by tile: the largest P of a tile is then 1, exact, and those next to it lie where bf16 is finest.  A
+// reference that lags the maximum (up to 2^8) saved 15% at 2048 tokens and cost up to 21% in the error against 64
+// bits; one reference for both tiles of a wave, up to 0.4%.  The scale in the exponent's fma with the denominator
+// from the rounded P saved 2 to 5% for 0 to 2% less error, but rounds 1 to 6% of the outputs the other way.
 // Every K/V block staged in LDS serves all waves.  Per block and wave:
 //   S^T = K Q^T   (per 32 keys x 32 queries 8 v_mfma_f32_32x32x16_bf16): with this orientation each
 //                 lane holds one query and 16 of its keys, so the row max and sum need one
@@ -47,10 +51,9 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 constexpr int kQH = 32, kKH = 8, kD = 128;
 constexpr int kBQ = 32;              // query tokens per workgroup
 constexpr int kKPad = kD + 8;        // K rows in LDS (bf16), padded
-constexpr float kSlack = 8.f;        // log2 a score may pass its query's reference by
 
-// Workgroup shape: HPW query heads of one KV head, KS waves per head, wave kq taking the 32 SUB-key
-// part kq of every block of 32 SUB KS keys.
+// Workgroup shape: HPW query heads of one KV head, KS waves per head, wave kq taking the 32-key tiles
+// kq + KS i (i < SUB) of every block of 32 SUB KS keys.
 template <int HPW, int KS, int SUB>
 struct Tile {
     static constexpr int kWaves = HPW * KS, kThreads = 64 * kWaves;
@@ -165,9 +168,9 @@ __global__ __launch_bounds__(64 * HPW * KS, 1) void prefill_attention_kernel(
         __syncthreads();
         const uint16_t(*ks)[kKPad] = stage_k(b & 1);
         const uint16_t(*vt)[VPAD] = stage_v(b & 1);
-        const int part = 32 * SUB * kq;      // this wave's keys of the block
-        if (BK * b + part <= last) {         // else every one of them is masked
-            // S^T, SUB tiles of 32 keys
+        const int part = 32 * kq;     // this wave's first tile of the block
+        if (BK * b + part <= last) {  // else every one of its keys is masked
+            // S^T, SUB tiles of 32 keys, 32 KS apart
             f32x16_t s[SUB];
 #pragma unroll
             for (int i = 0; i < SUB; ++i) s[i] = f32x16_t{};
@@ -175,59 +178,60 @@ __global__ __launch_bounds__(64 * HPW * KS, 1) void prefill_attention_kernel(
             for (int kk = 0; kk < 8; ++kk)
 #pragma unroll
                 for (int i = 0; i < SUB; ++i) {
-                    const bf16x8_t kf = *reinterpret_cast<const bf16x8_t*>(&ks[part + 32 * i + ql][16 * kk + 8 * half]);
+                    const bf16x8_t kf = *reinterpret_cast<const bf16x8_t*>(&ks[part + 32 * KS * i + ql][16 * kk + 8 * half]);
                     s[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[kk], s[i], 0, 0, 0);
                 }
-            // element e of tile i: key BK b + part + 32 i + 8 (e / 4) + 4 half + e % 4, query ql
+            // element e of tile i: key BK b + part + 32 KS i + 8 (e / 4) + 4 half + e % 4, query ql
             if (b >= first_masked) {
 #pragma unroll
                 for (int i = 0; i < SUB; ++i)
 #pragma unroll
                     for (int e = 0; e < 16; ++e) {
-                        const int key = BK * b + part + 32 * i + 8 * (e >> 2) + 4 * half + (e & 3);
+                        const int key = BK * b + part + 32 * KS * i + 8 * (e >> 2) + 4 * half + (e & 3);
                         s[i][e] = key <= qpos ? s[i][e] : -INFINITY;
                     }
             }
-            float bmax = fmaxf(s[0][0], s[0][1]);
+            // tile by tile: the reference m of a query is its largest score so far (-inf: no key of this
+            // wave visible yet, every P is 0)
 #pragma unroll
-            for (int e = 2; e < 16 * SUB; e += 2) bmax = fmaxf(fmaxf(bmax, s[e >> 4][e & 15]), s[e >> 4][(e & 15) + 1]);
-            bmax = max_xor32(bmax) * c;  // with the other 32-lane half's keys of the same query rows
-            // the reference m only has to keep exp2(s c - m) in range: it moves up, and the sums with it,
-            // when some query of the wave passes it by 2^8 (its first visible key among them)
-            if (__any(bmax > m + kSlack)) {
+            for (int i = 0; i < SUB; ++i) {
+                float bmax = fmaxf(s[i][0], s[i][1]);
+#pragma unroll
+                for (int e = 2; e < 16; e += 2) bmax = fmaxf(fmaxf(bmax, s[i][e]), s[i][e + 1]);
+                bmax = max_xor32(bmax) * c;  // with the other 32-lane half's keys of the same query rows
                 const float mn = fmaxf(m, bmax);
-                const float alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+                const float mr = mn == -INFINITY ? 0.f : mn;
+                const float alpha = __builtin_amdgcn_exp2f(m - mr);
                 m = mn;
-                l *= alpha;
+                float bsum = 0.f;
+                bf16x8_t pf[2];
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                for (int u = 0; u < 2; ++u)
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) o[i][e] *= alpha;
-            }
-            const float mr = m == -INFINITY ? 0.f : m;  // no key of this wave visible yet: every P is 0
-            float bsum = 0.f;
-            bf16x8_t pf[2 * SUB];
+                    for (int v = 0; v < 8; ++v) {
+#pragma clang fp contract(off)
+                        const float p = __builtin_amdgcn_exp2f(s[i][8 * u + v] * c - mr);
+                        bsum += p;
+                        pf[u][v] = (__bf16)p;
+                    }
+                l = l * alpha + sum_xor32(bsum);
 #pragma unroll
-            for (int u = 0; u < 2 * SUB; ++u)
+                for (int d = 0; d < 4; ++d)
 #pragma unroll
-                for (int v = 0; v < 8; ++v) {
-                    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u >> 1][8 * (u & 1) + v], c, -mr));
-                    bsum += p;
-                    pf[u][v] = (__bf16)p;
-                }
-            l += sum_xor32(bsum);
-            // O^T += V^T P^T: K step u covers keys part + 16 u + {4 half + 0..3, 8 + 4 half + 0..3}
+                    for (int e = 0; e < 16; ++e) o[d][e] *= alpha;
+                // O^T += V^T P^T: K step u covers keys .. + 16 u + {4 half + 0..3, 8 + 4 half + 0..3} of the tile
 #pragma unroll
-            for (int u = 0; u < 2 * SUB; ++u) {
-                const int key = part + 16 * u + 4 * half;
+                for (int u = 0; u < 2; ++u) {
+                    const int key = part + 32 * KS * i + 16 * u + 4 * half;
 #pragma unroll
-                for (int dt = 0; dt < 4; ++dt) {
-                    const uint16_t* row = vt[32 * dt + ql];
-                    const uint2 a0 = *reinterpret_cast<const uint2*>(row + vt_col(32 * dt, key));
-                    const uint2 a1 = *reinterpret_cast<const uint2*>(row + vt_col(32 * dt, key + 8));
-                    const uint4 av = make_uint4(a0.x, a0.y, a1.x, a1.y);
-                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, av), pf[u], o[dt],
-                                                                    0, 0, 0);
+                    for (int dt = 0; dt < 4; ++dt) {
+                        const uint16_t* row = vt[32 * dt + ql];
+                        const uint2 a0 = *reinterpret_cast<const uint2*>(row + vt_col(32 * dt, key));
+                        const uint2 a1 = *reinterpret_cast<const uint2*>(row + vt_col(32 * dt, key + 8));
+                        const uint4 av = make_uint4(a0.x, a0.y, a1.x, a1.y);
+                        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, av), pf[u], o[dt],
+                                                                        0, 0, 0);
+                    }
                 }
             }
         }
@@ -337,8 +341,10 @@ MOSS_API int moss_prefill_attention(const void* q, const void* k_cache, const vo
     // workgroups per 32 tokens), then 4 heads x 2 key parts.  Measured on MI355X at start 0 (and
     // after a cached prefix), against 4 heads x 2 parts: 128 / 256 / 512 tokens in 7.4 / 9.5 /
     // 14.1 us against 9.3 / 12.2 / 18.9, 128 after 1900 rows in 34 against 53; 1024 and 2048 tokens
-    // in 31 / 106 us against 40 / 117 with 2 heads x 4 parts (both with 32-key parts and the earlier
-    // softmax; today's times are at the head of this file)
+    // in 31 / 106 us against 40 / 117 with 2 heads x 4 parts (all with 32-key parts and a test around every
+    // load; today's times are at the head of this file).  Two tiles a wave: 4 heads x 2 parts of one tile take
+    // 17.2 / 28.5 / 98.4 us at 513 / 1024 / 2048 tokens where two take 16.0 / 25.9 / 86.3 (both with the scale in
+    // the exponent's fma)
     if (n <= 512)
         launch_prefill<2, 4, 1>(q, k_cache, v_cache, start, out, n, L, (hipStream_t)stream);
     else
