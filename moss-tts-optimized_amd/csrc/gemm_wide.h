@@ -25,7 +25,8 @@ enum WideEpilogue { kWidePlain = 0, kWideSplit = 1, kWideSilu = 2, kWideQkRope =
 // Tile and K split of one call: 128 r weight rows x 32 jt tokens per workgroup, split workgroups per tile.
 struct WidePlan {
     int r, jt, split;
-    bool any;  // the form for any K % 64 == 0 and any N
+    bool any;   // the form for any K % 64 == 0 and any N
+    double us;  // expected time
 };
 
 struct WideArgs {
@@ -41,8 +42,9 @@ struct WideArgs {
 // K % 64 == 0 and any N; nw: weight rows.
 bool wide_shape(int fmt, int K, int nw);
 bool wide_any_shape(int fmt, int K, int nw);
-// The tile and split with the least expected time; max_split 1 keeps K whole.
-WidePlan wide_plan(int fmt, int M, int K, int nw, int max_split);
+// The tile and split with the least expected time, min_split <= split <= max_split (powers of two; 1 and 1: K
+// whole).
+WidePlan wide_plan(int fmt, int M, int K, int nw, int min_split, int max_split);
 // The form for any K % 64 == 0 and any N of the plan above, for operands without the regular one's alignment.
 WidePlan wide_plan_any(int fmt, int M, int K, int nw, int max_split);
 int wide_launch_w4(WideEpilogue epi, const WidePlan& p, const WideArgs& a, hipStream_t st);

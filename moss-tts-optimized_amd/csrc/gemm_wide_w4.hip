@@ -69,9 +69,8 @@ bool wide_shape(int fmt, int K, int nw) {
 // two of 512 x 4096.  A split leaves every workgroup at least two blocks of K and its partials fit 32 MiB.  The any-shape form, a few percent slower a step, is also
 // weighed where the regular one fits: it splits a K of any number of steps (e4m3 K = 6400 = 100 steps, M =
 // 10, N = 3000: 31.8 us whole, 11.4 split).
-static WidePlan plan(int fmt, int M, int K, int nw, int max_split, bool regular) {
-    WidePlan best{1, 1, 1, !regular};
-    double least = 1e30;
+static WidePlan plan(int fmt, int M, int K, int nw, int min_split, int max_split, bool regular) {
+    WidePlan best{1, 1, 1, !regular, 1e30};
     const double wbytes = (double)nw * K * (fmt == kInt4G32 ? 0.5625 : 1.0);
     const int total = K / kStep;
     for (int r = 1; r <= 2; ++r)
@@ -79,7 +78,7 @@ static WidePlan plan(int fmt, int M, int K, int nw, int max_split, bool regular)
             const StepCost& c = kStepCost[fmt][r - 1];
             if (!c.alone[jt - 1] || (jt > 1 && 32 * (jt - 1) >= M)) continue;
             const long tiles = (long)((M + 32 * jt - 1) / (32 * jt)) * ((nw + 128 * r - 1) / (128 * r));
-            for (int split = 1; split <= max_split; split *= 2) {
+            for (int split = min_split; split <= max_split; split *= 2) {
                 const bool any = !regular || total % (4 * split);  // the regular form: whole blocks of four steps
                 if (any && !any_tile(r, jt)) break;
                 const int steps = any ? ((total + split - 1) / split + 3) & ~3 : total / split;
@@ -88,20 +87,17 @@ static WidePlan plan(int fmt, int M, int K, int nw, int max_split, bool regular)
                 const double ns = (any ? 1.06 : 1.0) * (per_cu == 1 ? c.alone[jt - 1] : (double)per_cu * c.shared[jt - 1]);
                 double us = 3.5 + std::max(steps * ns / 1000, wbytes / 4.5e6);
                 if (split > 1) us += 2.0 + (double)split * M * nw * 8 / 8e6;
-                if (us < least) {
-                    least = us;
-                    best = {r, jt, split, any};
-                }
+                if (us < best.us) best = {r, jt, split, any, us};
             }
         }
     return best;
 }
 
-WidePlan wide_plan(int fmt, int M, int K, int nw, int max_split) {
-    return plan(fmt, M, K, nw, max_split, wide_shape(fmt, K, nw));
+WidePlan wide_plan(int fmt, int M, int K, int nw, int min_split, int max_split) {
+    return plan(fmt, M, K, nw, min_split, max_split, wide_shape(fmt, K, nw));
 }
 
-WidePlan wide_plan_any(int fmt, int M, int K, int nw, int max_split) { return plan(fmt, M, K, nw, max_split, false); }
+WidePlan wide_plan_any(int fmt, int M, int K, int nw, int max_split) { return plan(fmt, M, K, nw, 1, max_split, false); }
 
 int wide_launch_w4(WideEpilogue epi, const WidePlan& p, const WideArgs& a, hipStream_t st) {
     switch (10 * p.r + p.jt) {

@@ -907,8 +907,8 @@ bool reg_tile_shape(int K, int N, bool int4) {
     return int4 && N % 4 == 0 && (K / kBK) % kTs == 0 && G % 16 == 0 && (G % 128) % 16 == 0;
 }
 
-// The K split of the 128-token copy tile (bm: the token depth its split is counted with), which also
-// bounds the wide tile's above 64 tokens (wide_max_split).  M > 64 (MFMA-bound): split K (2..8,
+// The K split of the 128-token copy tile (bm: the token depth its split is counted with), which the
+// wide tile mostly keeps above 64 tokens (wide_choice).  M > 64 (MFMA-bound): split K (2..8,
 // >= 2 blocks each) while the doubled workgroup count still fits one per CU.  M <= 64 (bound by
 // the weight stream): split while the workgroups fit two per CU and the fp32 partials (written
 // and read back once) stay below half the weight bytes.  Shapes it does not take use the LDS
@@ -940,8 +940,23 @@ Plan plan_gemm(int M, int K, int N, bool int4) {
     }
 }
 
-int wide_max_split(int fmt, int M, int K, int N) {
-    return fmt == kInt4G32 && M > 64 && reg_tile_shape(K, N, true) && plan_gemm(M, K, N, true).split == 1 ? 1 : 16;
+// The wide tile's plan.  INT4 above 64 tokens: plan_gemm's split, so that a sum keeps its order (the fused
+// epilogues run without a workspace where that is 1, and the plain GEMM of the same shape sums alike), unless
+// it is not 1 and another split is expected to take 15% less.  A sum in another order rounds to another bf16 in
+// a few of 10^4 outputs, which the rest of a layer spreads to 0.0024 of its output.  Keeping it costs one layer of
+// 150 tokens 1.4% (137.3 -> 139.1 us: q||k||v in two shares for four, down in four for eight); M = 301 down,
+// expected at 40 us in four shares for 49 in two, takes four.
+WidePlan wide_choice(int fmt, int M, int K, int N) {
+    const WidePlan best = wide_plan(fmt, M, K, N, 1, 16);
+    if (fmt != kInt4G32 || M <= 64 || !reg_tile_shape(K, N, true)) return best;
+    const int split = plan_gemm(M, K, N, true).split;
+    const WidePlan kept = wide_plan(fmt, M, K, N, split, split);
+    return split == 1 || kept.us * 0.85 <= best.us ? kept : best;
+}
+
+WidePlan wide_choice_any(int fmt, int M, int K, int N) {
+    const bool whole = fmt == kInt4G32 && M > 64 && reg_tile_shape(K, N, true) && plan_gemm(M, K, N, true).split == 1;
+    return wide_plan_any(fmt, M, K, N, whole ? 1 : 16);
 }
 
 Plan plan_lds(int M, int K, int N) {
@@ -1036,9 +1051,7 @@ bool stream_better(int fmt, int M, int K, int N) {
 
 // Whether the wide tile (gemm_wide_kernel.h) takes a call, and how.  Shapes without whole blocks of K or
 // quads of N and misaligned pointers take its any-shape form (INT4 M = 150, K = 4160, N = 1001: 36.9 -> 18.0 us
-// against the LDS tiles, M = 600, K = 11008, N = 4100: 158 -> 111).  Above 64 INT4 tokens it splits K
-// only where plan_gemm does: there the fused epilogues run without a workspace, and the plain GEMM
-// of the same shape sums in the same order.  A call whose planned split finds no workspace goes to the
+// against the LDS tiles, M = 600, K = 11008, N = 4100: 158 -> 111).  A call whose planned split finds no workspace goes to the
 // weight-streaming kernel if that takes it (K = N = 4096, M = 24: 10 us against 24 us unsplit).
 bool choose_wide(int fmt, int M, int K, int N, const void* x, const void* qw, const void* sc, const void* zp,
                  const void* y, const void* ws, long long ws_bytes, WidePlan& p) {
@@ -1050,13 +1063,10 @@ bool choose_wide(int fmt, int M, int K, int N, const void* x, const void* qw, co
     if (any && fmt == kInt4G32 && N % 4 && M > 32 && M <= 64 && K < 768) return false;
     const bool stream = stream_shape(fmt, M, K, N, x, qw, sc, zp, y);
     if (stream && stream_better(fmt, M, K, N)) return false;
-    auto plan = [&](int max_split) {
-        return any ? wide_plan_any(fmt, M, K, N, max_split) : wide_plan(fmt, M, K, N, max_split);
-    };
-    p = plan(wide_max_split(fmt, M, K, N));
+    p = any ? wide_choice_any(fmt, M, K, N) : wide_choice(fmt, M, K, N);
     if (split_fits(p.split, ws, ws_bytes, y, M, N)) return true;
     if (stream) return false;
-    p = plan(1);
+    p = any ? wide_plan_any(fmt, M, K, N, 1) : wide_plan(fmt, M, K, N, 1, 1);
     return true;
 }
 
@@ -1141,7 +1151,7 @@ long long gemm_workspace_bytes(int M, int K, int N) {
         if (p.split > 1) bytes = std::max(bytes, (long long)p.split * M * N * 4);
     for (int fmt : {(int)kInt4G32, (int)kFp8E4M3})
         if (wide_any_shape(fmt, K, N)) {
-            const int split = wide_plan(fmt, M, K, N, wide_max_split(fmt, M, K, N)).split;
+            const int split = wide_choice(fmt, M, K, N).split;
             if (split > 1) bytes = std::max(bytes, (long long)split * M * N * 4);
         }
     return bytes;
@@ -1182,7 +1192,7 @@ MOSS_API int moss_w4g32_gemm_silu(const void* x, const void* qw, const void* sc,
     hipStream_t st = (hipStream_t)stream;
     if (silu_fusable_shape(M, K, N) && MOSS_ALIGNED(y, 8) && MOSS_ALIGNED(sc, 16) && MOSS_ALIGNED(zp, 8)) {
         if (wide_shape(kInt4G32, K, 2 * N))
-            return wide_launch_w4(kWideSilu, wide_plan(kInt4G32, M, K, 2 * N, 1),
+            return wide_launch_w4(kWideSilu, wide_plan(kInt4G32, M, K, 2 * N, 1, 1),
                                   WideArgs{x, qw, sc, zp, nullptr, y, nullptr, M, K, N, QkRope{}}, st);
         const dim3 grid((unsigned)(((M + 127) / 128) * ((N + 63) / 64)));
         hipLaunchKernelGGL((w4g32_gemm_tdma_kernel<false, true>), grid, dim3(256), 0, st, (const uint16_t*)x,
@@ -1240,7 +1250,7 @@ MOSS_API int moss_w4g32_gemm_qk_rope(const void* x, const void* qw, const void* 
                         (const uint16_t*)sin, (uint16_t*)k_cache, (uint16_t*)v_cache, (const int64_t*)positions, L,
                         eps};
         if (wide_shape(kInt4G32, K, kQkvN))
-            return wide_launch_w4(kWideQkRope, wide_plan(kInt4G32, M, K, kQkvN, 1),
+            return wide_launch_w4(kWideQkRope, wide_plan(kInt4G32, M, K, kQkvN, 1, 1),
                                   WideArgs{x, qw, sc, zp, nullptr, q_out, nullptr, M, K, kQkvN, qr}, st);
         const dim3 grid((unsigned)(((M + 127) / 128) * (kQkvN / 128)));
         hipLaunchKernelGGL((w4g32_gemm_tdma_kernel<false, false, true>), grid, dim3(256), 0, st, (const uint16_t*)x,

@@ -38,7 +38,8 @@ static std::vector<char> operand(size_t bytes) {
 }
 
 static int runs;
-static bool check(int fmt, WidePlan p, WideEpilogue epi, int M, int N, int K) {
+static bool check(int fmt, int r, int jt, int split, bool any, WideEpilogue epi, int M, int N, int K) {
+    const WidePlan p{r, jt, split, any, 0};
     const int nw = epi == kWideSilu ? 2 * N : N, G = K / 32, L = 64, before = (int)violations;
     const bool int4 = fmt == kInt4G32;
     operands.clear();
@@ -70,17 +71,17 @@ static bool bounds() {
             // one row past a tile, rows that end in its first and in its second row tile, one short of it
             for (int n : {4, 124, 128, 132, 252, 256, bn + 4, bn + 128, bn + 132, 2 * bn - 4}) {
                 const int m = 32 * jt + 1;
-                ok &= check(fmt, {r, jt, 1, false}, kWidePlain, m, n, 512);
-                ok &= check(fmt, {r, jt, 2, false}, kWideSplit, m, n, 512);
-                if (fmt == kInt4G32) ok &= check(fmt, {r, jt, 1, false}, kWideSilu, m, n, 512);
+                ok &= check(fmt, r, jt, 1, false, kWidePlain, m, n, 512);
+                ok &= check(fmt, r, jt, 2, false, kWideSplit, m, n, 512);
+                if (fmt == kInt4G32) ok &= check(fmt, r, jt, 1, false, kWideSilu, m, n, 512);
             }
-            if (fmt == kInt4G32) ok &= check(fmt, {r, jt, 1, false}, kWideQkRope, 32 * jt - 1, 6144, 512);
+            if (fmt == kInt4G32) ok &= check(fmt, r, jt, 1, false, kWideQkRope, 32 * jt - 1, 6144, 512);
             if (r == 1 ? jt == 3 : jt != 4) continue;  // no any-shape instance
             for (int n : {1, 127, 128, 129, 255, bn + 1, bn + 128, 2 * bn - 1})
                 for (int k : {64, 576}) {
-                    ok &= check(fmt, {r, jt, 1, true}, kWidePlain, 32 * jt - 1, n, k);
+                    ok &= check(fmt, r, jt, 1, true, kWidePlain, 32 * jt - 1, n, k);
                     // shares of K past its end among them
-                    for (int split : {2, 4}) ok &= check(fmt, {r, jt, split, true}, kWideSplit, 33, n, k);
+                    for (int split : {2, 4}) ok &= check(fmt, r, jt, split, true, kWideSplit, 33, n, k);
                 }
         }
     printf("%d launches\n", runs);
@@ -93,10 +94,10 @@ int main(int argc, char** argv) {
     int fmt, M, K, N;
     const void* p = (const void*)4096;  // aligned for everything, never read
     while (scanf("%d %d %d %d", &fmt, &M, &K, &N) == 4) {
-        WidePlan w{0, 0, 0, false};
+        WidePlan w{};
         const long long ws = gemm_workspace_bytes(M, K, N);
         if (!(fmt == kInt4G32 && tokens_gemv(M, K, p, p))) {
-            if (!choose_wide(fmt, M, K, N, p, p, p, p, p, p, ws, w)) w = WidePlan{0, 0, 0, false};
+            if (!choose_wide(fmt, M, K, N, p, p, p, p, p, p, ws, w)) w = WidePlan{};
         }
         printf("%d %d %d %d %lld\n", w.r, w.jt, w.split, (int)w.any, ws);
     }

@@ -56,3 +56,19 @@ def test_offsets_fit_32_bits(gemm_wide_check):
     calls = [(f, 160, k, 4) for f in (0, 1) for k in (last, last + 256, 2 ** 24)]
     calls += [(0, 160, 4096, 2 ** 20 - 4), (0, 160, 4096, 2 ** 20), (1, 160, 4096, 2 ** 19 - 4), (1, 160, 4096, 2 ** 19)]
     assert [p[0] > 0 for p in _plans(gemm_wide_check, calls)] == [True, False, False] * 2 + [True, False] * 2
+
+
+def _earlier_split(m, k, n):
+    """The K shares of the 128-token INT4 tile, which the sums above 64 tokens have always had."""
+    tiles, steps, split = -(-m // 128) * (n // 128), k // 64, 1
+    while split < 8 and tiles * split * 2 <= 256 and steps % (8 * split) == 0 and steps // (2 * split) >= 8:
+        split *= 2
+    return split
+
+
+def test_sums_keep_their_order(gemm_wide_check):
+    """Above 64 tokens the projections of the 4096 / 12288 model sum K in the shares they had, but for the down
+    projection of 257 to 320 tokens, where four for two is expected to save more than 15%."""
+    calls = [(0, m, k, n) for m in range(65, 1100) for k, n in ((4096, 6144), (4096, 4096), (4096, 24576), (12288, 4096))]
+    other = {c[1:] for c, p in zip(calls, _plans(gemm_wide_check, calls)) if p[2] != _earlier_split(*c[1:])}
+    assert other == {(m, 12288, 4096) for m in range(257, 321)}
