@@ -407,10 +407,51 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
         return;
     }
     // C[n][m] of a 32 x 32 tile: lane l, element e -> n row 8 (e / 4) + 4 (l / 32) + e % 4, m column
-    // l % 32; the four e of a quad are consecutive n (N % 4 == 0: a quad is all in range or all out)
-    const bool quads = !ANY || (N % 4 == 0 && (EPI == kWideSplit || reinterpret_cast<uintptr_t>(Y) % 8 == 0));
-    const bool pairs = N % 2 == 0 && (EPI == kWideSplit || reinterpret_cast<uintptr_t>(Y) % 4 == 0);
-    auto scaled = [&](float v, int n) { return !INT4 && row_scale ? v * row_scale[n] : v; };
+    // l % 32; the four e of a quad are consecutive n
+    if constexpr (ANY) {
+        if (N % 4 || (EPI == kWidePlain && reinterpret_cast<uintptr_t>(Y) % 8)) {
+            // No quads: a store of one value per lane would touch a row per lane, so each 128-row half of the tile goes through the LDS of the ring, fp32 by token row
+            // (row t in buffer (t / 8) % 4, 16-byte chunk c at c ^ (t & 31)), and leaves row by row
+            // (M = 595, K = 320, N = 12317: 32.2 -> 21.4 us; M = 150, K = 4160, N = 1001: 17.0 -> 14.0).
+            auto chunk = [&](int row, int c) {
+                const int b = (row >> 3) & 3;
+                uint16_t* x = b == 0 ? X0 : b == 1 ? X1 : b == 2 ? X2 : X3;
+                return reinterpret_cast<float*>(x) + ((row >> 5) * 8 + (row & 7)) * 128 + 4 * (c ^ (row & 31));
+            };
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                __syncthreads();
+#pragma unroll
+                for (int j = 0; j < JT; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        *reinterpret_cast<float4*>(chunk(32 * j + (lane & 31), 8 * wave + 2 * q + half)) = make_float4(
+                            acc[r][j][4 * q], acc[r][j][4 * q + 1], acc[r][j][4 * q + 2], acc[r][j][4 * q + 3]);
+                __syncthreads();
+                const int nr = n0 + 128 * r, nn = min(128, N - nr), rows = min(BM, M - m0);
+                if (nn <= 0) break;
+                const bool v0 = lane < nn, v1 = lane + 64 < nn;
+                float s0 = 1.f, s1 = 1.f;
+                if (!INT4 && EPI == kWidePlain && row_scale) {
+                    if (v0) s0 = row_scale[nr + lane];
+                    if (v1) s1 = row_scale[nr + 64 + lane];
+                }
+                for (int row = wave; row < rows; row += 4) {
+                    const float c0 = chunk(row, lane >> 2)[lane & 3], c1 = chunk(row, 16 + (lane >> 2))[lane & 3];
+                    const size_t o = (size_t)(m0 + row) * N + nr + lane;
+                    if constexpr (EPI == kWideSplit) {
+                        float* out = part + (size_t)z * M * N + o;
+                        if (v0) out[0] = c0;
+                        if (v1) out[64] = c1;
+                    } else {
+                        if (v0) Y[o] = f32_to_bf16(c0 * s0);
+                        if (v1) Y[o + 64] = f32_to_bf16(c1 * s1);
+                    }
+                }
+            }
+            return;
+        }
+    }
 #pragma unroll
     for (int j = 0; j < JT; ++j) {
         const int m = m0 + 32 * j + (lane & 31);
@@ -420,29 +461,10 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
 #pragma unroll
             for (int q = 0; q < (EPI == kWideSilu ? 2 : 4); ++q) {
                 const int n = n0 + (EPI == kWideSilu ? 64 * r + 16 * wave : 128 * r + 32 * wave) + 8 * q + 4 * half;
-                if (n >= N) continue;
+                if (n >= N) continue;  // N % 4 == 0: a quad is all in range or all out
                 const f32x16_t& c = acc[r][j];
                 const float v0 = c[4 * q], v1 = c[4 * q + 1], v2 = c[4 * q + 2], v3 = c[4 * q + 3];
-                if (ANY && !quads) {  // outputs one by one, or in pairs for an even N
-                    const float v[4] = {v0, v1, v2, v3};
-#pragma unroll
-                    for (int e = 0; e < 4; e += 2) {
-                        const size_t o = (size_t)m * N + n + e;
-                        if (pairs && n + e < N) {
-                            if constexpr (EPI == kWideSplit)
-                                *reinterpret_cast<float2*>(part + (size_t)z * M * N + o) = make_float2(v[e], v[e + 1]);
-                            else
-                                *reinterpret_cast<uint32_t*>(Y + o) = pack_bf16x2(scaled(v[e], n + e), scaled(v[e + 1], n + e + 1));
-                        } else if (!pairs) {
-#pragma unroll
-                            for (int i = 0; i < 2; ++i) {
-                                if (n + e + i >= N) continue;
-                                if constexpr (EPI == kWideSplit) part[(size_t)z * M * N + o + i] = v[e + i];
-                                else Y[o + i] = f32_to_bf16(scaled(v[e + i], n + e + i));
-                            }
-                        }
-                    }
-                } else if constexpr (EPI == kWideSplit) {
+                if constexpr (EPI == kWideSplit) {
                     *reinterpret_cast<float4*>(part + ((size_t)z * M + m) * N + n) = make_float4(v0, v1, v2, v3);
                 } else {
                     uint2 o;
