@@ -47,6 +47,9 @@ bool wide_any_shape(int fmt, int K, int nw);
 WidePlan wide_plan(int fmt, int M, int K, int nw, int min_split, int max_split);
 // The form for any K % 64 == 0 and any N of the plan above, for operands without the regular one's alignment.
 WidePlan wide_plan_any(int fmt, int M, int K, int nw, int max_split);
+// The expected time of a plan on the scale of the LDS tiles' (lds_us in w4g32_gemm.hip): e4m3, and INT4 in the
+// any-shape form.
+double wide_us(int fmt, int M, int K, int nw, const WidePlan& p);
 int wide_launch_w4(WideEpilogue epi, const WidePlan& p, const WideArgs& a, hipStream_t st);
 int wide_launch_fp8(WideEpilogue epi, const WidePlan& p, const WideArgs& a, hipStream_t st);
 

@@ -63,12 +63,40 @@ bool wide_shape(int fmt, int K, int nw) {
     return fmt == kFp8E4M3 || (G % 16 == 0 && (G % 128) % 16 == 0);
 }
 
-// The expected time of each tile and split is what the step costs above give for the workgroups per CU,
+// The expected time of a plan from timings of 15000 random shapes (2 to 1024 tokens, K = 256 .. 12288, N = 64 ..
+// 16384, weights from memory): microseconds to start and to end (base) and per step and round of 256
+// workgroups, the partial sums and their reduction, the output and the weights.  Within 4 to 6% of half of the
+// times and 15% of nine in ten.
+struct FitCost {
+    double base[2][5], step[2][5];         // [r - 1][jt - 1]; step 0: no such instance
+    double split, part, out, weights;      // part: per 8 bytes at 8 TB/s; out at 4 TB/s; weights at 4.5 TB/s
+};
+constexpr FitCost kFitAny[2] = {
+    {{{2.1, 3.2, 0, 3.6, 3.2}, {0, 0, 0, 5.6, 0}}, {{0.374, 0.430, 0, 0.564, 0.657}, {0, 0, 0, 1.045, 0}}, 2.5, 2.3, 1.4, 0.68},
+    {{{2.3, 3.0, 0, 3.2, 3.0}, {0, 0, 0, 4.3, 0}}, {{0.231, 0.264, 0, 0.417, 0.468}, {0, 0, 0, 0.791, 0}}, 2.4, 2.0, 2.4, 0.51},
+};
+constexpr FitCost kFitFp8 = {{{2.2, 2.5, 2.2, 1.5, 2.0}, {0, 0, 2.9, 3.8, 3.4}},
+                             {{0.267, 0.300, 0.383, 0.461, 0.481}, {0, 0, 0.625, 0.721, 0.858}}, 2.0, 1.6, 2.6, 0.51};
+
+double wide_us(int fmt, int M, int K, int nw, const WidePlan& p) {
+    const FitCost& c = p.any ? kFitAny[fmt] : kFitFp8;
+    const int total = K / kStep;
+    const int steps = p.any ? ((total + p.split - 1) / p.split + 3) & ~3 : total / p.split;
+    const long wgs = (long)((M + 32 * p.jt - 1) / (32 * p.jt)) * ((nw + 128 * p.r - 1) / (128 * p.r)) * p.split;
+    const double mn = (double)M * nw;
+    double us = c.base[p.r - 1][p.jt - 1] + (double)((wgs + 255) / 256) * steps * c.step[p.r - 1][p.jt - 1] +
+                c.out * mn * 2 / 4e6 + c.weights * nw * K * (fmt == kInt4G32 ? 0.5625 : 1.0) / 4.5e6;
+    if (p.split > 1) us += c.split + c.part * p.split * mn * 8 / 8e6;
+    return us;
+}
+
+// The regular form: the expected time of each tile and split is what the step costs above give for the workgroups per CU,
 // not less than the weights' bytes at 4.5 TB/s, and for a split the partial sums written and read back
 // (8 bytes each at 8 TB/s: they mostly stay in the last-level cache) and the launch that adds them, 6 us for
-// two of 512 x 4096.  A split leaves every workgroup at least two blocks of K and its partials fit 32 MiB.  The any-shape form, a few percent slower a step, is also
-// weighed where the regular one fits: it splits a K of any number of steps (e4m3 K = 6400 = 100 steps, M =
-// 10, N = 3000: 31.8 us whole, 11.4 split).
+// two of 512 x 4096.  A split leaves a share two blocks of K and its partials fit 32 MiB.  The any-shape form, a
+// few percent slower a step, is also weighed where the regular one fits: it splits a K of any number of steps
+// (e4m3 K = 6400 = 100 steps, M = 10, N = 3000: 31.8 us whole, 11.4 split).  Its shares are whole blocks, so the
+// last ones can lie past K and add zeros (65 steps split by 8: shares of 12 steps, the last two empty).
 static WidePlan plan(int fmt, int M, int K, int nw, int min_split, int max_split, bool regular) {
     WidePlan best{1, 1, 1, !regular, 1e30};
     const double wbytes = (double)nw * K * (fmt == kInt4G32 ? 0.5625 : 1.0);
@@ -84,6 +112,12 @@ static WidePlan plan(int fmt, int M, int K, int nw, int min_split, int max_split
                 const int steps = any ? ((total + split - 1) / split + 3) & ~3 : total / split;
                 if (split > 1 && (steps < 8 || (long long)split * M * nw * 4 > 32ll << 20)) break;
                 const long per_cu = (tiles * split + 255) / 256;
+                if (!regular) {
+                    const WidePlan p{r, jt, split, true, 0};
+                    const double us = wide_us(fmt, M, K, nw, p);
+                    if (us < best.us) best = {r, jt, split, true, us};
+                    continue;
+                }
                 const double ns = (any ? 1.06 : 1.0) * (per_cu == 1 ? c.alone[jt - 1] : (double)per_cu * c.shared[jt - 1]);
                 double us = 3.5 + std::max(steps * ns / 1000, wbytes / 4.5e6);
                 if (split > 1) us += 2.0 + (double)split * M * nw * 8 / 8e6;

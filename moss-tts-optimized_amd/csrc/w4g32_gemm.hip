@@ -11,10 +11,11 @@
 // epilogue (src/moss_tts/_runtime/fused_mlp.py:20-21).  The fp8 MFMA forms are not used:
 // they would round the bf16 activations to e4m3 as well.
 //
-// Both formats take the wide tile (gemm_wide_kernel.h) wherever its shape conditions hold
-// (wide_shape) and the few-token paths below do not win (choose_wide).  w4g32_gemm_tdma_kernel, the
-// 128-token tile with 64-bit addresses, takes INT4 weights past 32-bit offsets; other shapes and
-// misaligned scale or zero-point pointers take the LDS tiles:
+// Both formats take the wide tile (gemm_wide_kernel.h) wherever its operands lie within 32-bit offsets and
+// it is expected to be the fastest (choose_wide); w4g32_gemm_tdma_kernel, the 128-token tile with 64-bit
+// addresses, takes regular INT4 shapes past those offsets.  The rest take the LDS tiles: what the wide tile
+// is slower at (a short K or many rows of 33 to 64 tokens, without whole blocks of K or quads of N, with
+// misaligned pointers, or e4m3), and e4m3 and other INT4 shapes past 32-bit offsets:
 //
 // LDS tiles: BM x BN outputs (BM, BN in {64, 128}) per 256-thread workgroup, 2 x 2 waves of
 // (BM/2) x (BN/2), K in steps of 64 (two quantization groups).  Pipeline: two LDS buffers and
@@ -977,6 +978,26 @@ Plan plan_lds(int M, int K, int N) {
     return p;
 }
 
+// The expected time of an LDS plan, fitted like wide_us to the same shapes: within 1.4 (INT4) and 3.7% (e4m3) of
+// half of the times and 5 and 11% of nine in ten.
+double lds_us(int fmt, int M, int K, int N, const Plan& p) {
+    struct Cost {
+        double base[2], step[2];  // one round of workgroups; more
+    };
+    static constexpr Cost kCost[2][3] = {  // 64 x 64, 128 x 64 and 64 x 128, 128 x 128 tiles
+        {{{2.8, 2.5}, {0.354, 0.295}}, {{3.8, 4.9}, {0.495, 0.486}}, {{2.9, 1.9}, {0.782, 0.664}}},
+        {{{3.6, 4.8}, {0.231, 0.185}}, {{6.1, 7.4}, {0.367, 0.333}}, {{5.8, 5.0}, {0.627, 0.539}}},
+    };
+    static constexpr double kSplit[2] = {2.1, 1.5}, kPart[2] = {2.2, 0.92}, kOut[2] = {1.6, 2.9}, kWeights[2] = {0.37, 0.21};
+    const Cost& c = kCost[fmt][p.bm == 64 && p.bn == 64 ? 0 : p.bm == 128 && p.bn == 128 ? 2 : 1];
+    const long wgs = (long)((M + p.bm - 1) / p.bm) * ((N + p.bn - 1) / p.bn) * p.split, rounds = (wgs + 255) / 256;
+    const double mn = (double)M * N;
+    double us = c.base[rounds > 1] + (double)rounds * (K / kBK / p.split) * c.step[rounds > 1] + kOut[fmt] * mn * 2 / 4e6 +
+                kWeights[fmt] * N * K * (fmt == kInt4G32 ? 0.5625 : 1.0) / 4.5e6;
+    if (p.split > 1) us += kSplit[fmt] + kPart[fmt] * p.split * mn * 8 / 8e6;
+    return us;
+}
+
 template <int BM, int BN, int FMT, bool TAIL>
 void launch_tile2(const Plan& p, const void* x, const void* qw, const void* sc, const void* zp, void* y, void* part,
                   int M, int K, int N, const float* row_scale, hipStream_t st) {
@@ -1038,36 +1059,46 @@ bool split_fits(int split, const void* ws, long long ws_bytes, const void* y, in
 }
 
 // Where the weight-streaming kernel, which never splits K over workgroups, still beats the wide tile with
-// its partial sums: at most 256 workgroups (N <= 4096) and few activations to read in each (INT4 K = N =
-// 4096: M = 5 6.4 against 7.8 us, 16 8.2 / 8.9, 24 10.4 / 9.9; N = 6144, M = 6 11.3 / 10.2; e4m3 M = 2 6.1 /
-// 8.3, 16 8.3 / 9.2; K = 12288, M = 4 13.2 / 13.6, 8 15.5 / 13.9), and for e4m3, whose tile has no fewer
-// bytes to hide its steps behind, very few tokens or very many rows (N = 12288: M = 3 12.7 / 15.0, 12 17.5 /
-// 15.1; N = 24576: M = 5 27.0 / 34.7, 12 32.8 / 34.7, 16 36.2 / 35.2).
+// its partial sums: few activations to read in each workgroup (M K), by the format and for up to one workgroup
+// per CU (N <= 4096) or more.  Streamed / wide, us, weights from memory:
+//   INT4 N = 4096: K = 4096 M = 16 7.8 / 8.9, 21 9.6 / 9.4, 24 10.2 / 9.6; K = 12288 M = 6 14.3 / 15.7, 7 15.1 / 15.8,
+//        8 15.6 / 15.8, 12 17.3 / 16.0;  N = 6144: M = 5 10.6 / 10.2, 8 11.8 / 10.4
+//   e4m3 N = 4096, K = 12288: M = 6 14.4 / 17.6, 12 17.4 / 17.8, 14 18.2 / 17.7;  N = 6144: M = 6 10.6 / 11.7, 12 12.3 / 12.1;
+//        N = 12288: M = 6 16.0 / 18.7, 12 17.7 / 19.1, 15 18.8 / 19.1;  N = 24576: M = 12 32.7 / 32.7, 14 33.7 / 32.4
 bool stream_better(int fmt, int M, int K, int N) {
     const long long mk = (long long)M * K;
-    if (N <= 4096) return mk <= 16 * 4096;
-    return fmt == kFp8E4M3 && mk <= (N >= 16384 ? 12 : 5) * 4096;
+    if (N <= 4096) return mk <= (fmt == kInt4G32 ? 21 : 38) * 4096;
+    return fmt == kFp8E4M3 && mk <= 13 * 4096;
 }
 
 // Whether the wide tile (gemm_wide_kernel.h) takes a call, and how.  Shapes without whole blocks of K or
-// quads of N and misaligned pointers take its any-shape form (INT4 M = 150, K = 4160, N = 1001: 36.9 -> 18.0 us
-// against the LDS tiles, M = 600, K = 11008, N = 4100: 158 -> 111).  A call whose planned split finds no workspace goes to the
-// weight-streaming kernel if that takes it (K = N = 4096, M = 24: 10 us against 24 us unsplit).
+// quads of N and misaligned pointers take its any-shape form, e4m3 the regular one too, where it is expected to
+// take less time than the LDS tiles.  A short K, whose steps the any-shape form rounds up to a block of four, and
+// 33 to 64 tokens over many rows stay in those (M = 424, K = 832, N = 11701: 22.4 us there, 34.6 in the wide
+// tile; e4m3 M = 53, K = 1536, N = 13434: 11.6, 16.5).  40000 random calls (INT4 and e4m3, M = 2 .. 1024, K = 256 ..
+// 12288, N = 64 .. 16384) take 0.67 of the time they took in the LDS tiles and the streaming kernel in the mean, and
+// 0.2% of them over 1.05 times; with the wide tile wherever it can run 7% did.  A plan whose partial sums do not
+// fit the workspace is split less, or left to the streaming kernel where that takes the shape (K = N = 4096, M =
+// 24: 10 us against 24 us unsplit).
 bool choose_wide(int fmt, int M, int K, int N, const void* x, const void* qw, const void* sc, const void* zp,
                  const void* y, const void* ws, long long ws_bytes, WidePlan& p) {
     const bool aligned = MOSS_ALIGNED(y, 8) && (fmt == kFp8E4M3 || (MOSS_ALIGNED(sc, 16) && MOSS_ALIGNED(zp, 8)));
     const bool any = !(wide_shape(fmt, K, N) && aligned);
     if (any && !(wide_any_shape(fmt, K, N) && MOSS_ALIGNED(sc, 2))) return false;
-    // a K of a few steps at 33 .. 64 tokens and N % 4 != 0 stays in the 64-token LDS tiles (M = 50, K = 320, N =
-    // 3001: 5.1 against 6.2 us; M = 40, K = 704, N = 16383: 7.7 / 8.7; K = 768: equal; M = 72, K = 256: 6.0 / 4.6)
-    if (any && fmt == kInt4G32 && N % 4 && M > 32 && M <= 64 && K < 768) return false;
     const bool stream = stream_shape(fmt, M, K, N, x, qw, sc, zp, y);
     if (stream && stream_better(fmt, M, K, N)) return false;
     p = any ? wide_choice_any(fmt, M, K, N) : wide_choice(fmt, M, K, N);
-    if (split_fits(p.split, ws, ws_bytes, y, M, N)) return true;
-    if (stream) return false;
-    p = any ? wide_plan_any(fmt, M, K, N, 1) : wide_plan(fmt, M, K, N, 1, 1);
-    return true;
+    while (!split_fits(p.split, ws, ws_bytes, y, M, N)) {
+        if (stream) return false;
+        p = any ? wide_plan_any(fmt, M, K, N, p.split / 2) : wide_plan(fmt, M, K, N, 1, p.split / 2);
+    }
+    if (stream || (fmt == kInt4G32 && !any)) return true;
+    Plan lds = plan_lds(M, K, N);
+    if (!split_fits(lds.split, ws, ws_bytes, y, M, N)) lds.split = 1;
+    // the any-shape form's time is known to 15% only, and the LDS tiles took these calls before; of the regular
+    // e4m3 ones they are as fast at about 50 tokens of K = N = 4096 (M = 60: 12.2 us, 13.3 in the wide tile) and of
+    // 12288 x 4096 (M = 33: 20.0, 19.1)
+    return wide_us(fmt, M, K, N, p) < (any ? 0.95 : 1.05) * lds_us(fmt, M, K, N, lds);
 }
 
 // The LDS tiles, and the 128-token copy tile for INT4 weights past the wide tile's 32-bit offsets;
