@@ -195,7 +195,8 @@ int moss_w4a8_norm_gateup_silu(const void *x, const void *res, const void *norm_
 /* ------------------------------------------------------------- prefill GEMM */
 /* Y bf16 [M, N] = X bf16 [M, K] . dequant(W)^T with W row-packed INT4-G32 (K % 64 == 0);
  * weights are dequantized bit-exactly (bf16_rne((q-z)*s)), in the registers that feed
- * the matrix cores (into LDS for a few short-K shapes and weights past 2 GiB), fp32 accumulate.  2 to 4 tokens (4 only for
+ * the matrix cores, or into LDS where that is faster (a short K, many rows of 33 to 64 tokens), fp32 accumulate.
+ * 2 to 4 tokens (4 only for
  * K <= 4096) take the multi-token GEMV of moss_w4g32_gemv instead (no matrix cores; each row of Y
  * equal to the single-token GEMV's).  When the output tiles alone
  * cannot fill the GPU the K dimension is split over workgroups: that needs a caller-owned fp32 workspace

@@ -41,7 +41,8 @@ struct WideArgs {
 // Shapes the tile takes: whole blocks of K and 4-output stores (the fused epilogues need them), or any
 // K % 64 == 0 and any N; nw: weight rows.
 bool wide_shape(int fmt, int K, int nw);
-bool wide_any_shape(int fmt, int K, int nw);
+bool wide_any_shape(int K);
+bool wide_silu_shape(int K, int N);  // the SiLU form, 2 N weight rows
 // The tile and split with the least expected time, min_split <= split <= max_split (powers of two; 1 and 1: K
 // whole).
 WidePlan wide_plan(int fmt, int M, int K, int nw, int min_split, int max_split);

@@ -49,19 +49,20 @@ int launch_tile(WideEpilogue epi, const WidePlan& p, const WideArgs& a, hipStrea
 
 }  // namespace
 
-// The weight, and the activations of the deepest tile (160 rows of 2 K bytes), lie within the 32-bit offsets
-// of the buffer instructions.
-bool wide_any_shape(int fmt, int K, int nw) {
-    return K % kStep == 0 && (long long)nw * K / (fmt == kInt4G32 ? 2 : 1) < 1ll << 31 && 320ll * K < 1ll << 32;
-}
+// A workgroup's own weight rows (256 of K bytes) and activation rows (160 of 2 K) lie within the 32-bit offsets of
+// the buffer instructions.
+bool wide_any_shape(int K) { return K % kStep == 0 && 320ll * K < 1ll << 32; }
 
 // Whole blocks of four K steps and 4-output stores; INT4: the 8 zero bytes of every block on one
 // nibble side of their 128-group chunk (the last chunk a multiple of 16 groups long).
 bool wide_shape(int fmt, int K, int nw) {
-    if (nw % 4 || K % (4 * kStep) || !wide_any_shape(fmt, K, nw)) return false;
+    if (nw % 4 || K % (4 * kStep) || !wide_any_shape(K)) return false;
     const int G = K / 32;
     return fmt == kFp8E4M3 || (G % 16 == 0 && (G % 128) % 16 == 0);
 }
+
+// A SiLU workgroup reaches from its gate rows to the up rows, N of K / 2 bytes further on.
+bool wide_silu_shape(int K, int N) { return wide_shape(kInt4G32, K, 2 * N) && (long long)N * K < 1ll << 31; }
 
 // The expected time of a plan from timings of 15000 random shapes (2 to 1024 tokens, K = 256 .. 12288, N = 64 ..
 // 16384, weights from memory): microseconds to start and to end (base) and per step and round of 256

@@ -11,11 +11,11 @@
 // epilogue (src/moss_tts/_runtime/fused_mlp.py:20-21).  The fp8 MFMA forms are not used:
 // they would round the bf16 activations to e4m3 as well.
 //
-// Both formats take the wide tile (gemm_wide_kernel.h) wherever its operands lie within 32-bit offsets and
-// it is expected to be the fastest (choose_wide); w4g32_gemm_tdma_kernel, the 128-token tile with 64-bit
-// addresses, takes regular INT4 shapes past those offsets.  The rest take the LDS tiles: what the wide tile
-// is slower at (a short K or many rows of 33 to 64 tokens, without whole blocks of K or quads of N, with
-// misaligned pointers, or e4m3), and e4m3 and other INT4 shapes past 32-bit offsets:
+// Both formats take the wide tile (gemm_wide_kernel.h) wherever its offsets fit 32 bits and it is expected to
+// be the fastest (choose_wide); w4g32_gemm_tdma_kernel, the 128-token tile with 64-bit addresses, takes the
+// fused gate||up of a weight past 2 GiB and K from 13.4 million on.  The rest take the LDS tiles: what the
+// wide tile is slower at (a short K or many rows of 33 to 64 tokens, without whole blocks of K or quads of N,
+// with misaligned pointers, or e4m3), and such a K:
 //
 // LDS tiles: BM x BN outputs (BM, BN in {64, 128}) per 256-thread workgroup, 2 x 2 waves of
 // (BM/2) x (BN/2), K in steps of 64 (two quantization groups).  Pipeline: two LDS buffers and
@@ -1084,7 +1084,7 @@ bool choose_wide(int fmt, int M, int K, int N, const void* x, const void* qw, co
                  const void* y, const void* ws, long long ws_bytes, WidePlan& p) {
     const bool aligned = MOSS_ALIGNED(y, 8) && (fmt == kFp8E4M3 || (MOSS_ALIGNED(sc, 16) && MOSS_ALIGNED(zp, 8)));
     const bool any = !(wide_shape(fmt, K, N) && aligned);
-    if (any && !(wide_any_shape(fmt, K, N) && MOSS_ALIGNED(sc, 2))) return false;
+    if (any && !(wide_any_shape(K) && MOSS_ALIGNED(sc, 2))) return false;
     const bool stream = stream_shape(fmt, M, K, N, x, qw, sc, zp, y);
     if (stream && stream_better(fmt, M, K, N)) return false;
     p = any ? wide_choice_any(fmt, M, K, N) : wide_choice(fmt, M, K, N);
@@ -1101,7 +1101,7 @@ bool choose_wide(int fmt, int M, int K, int N, const void* x, const void* qw, co
     return wide_us(fmt, M, K, N, p) < (any ? 0.95 : 1.05) * lds_us(fmt, M, K, N, lds);
 }
 
-// The LDS tiles, and the 128-token copy tile for INT4 weights past the wide tile's 32-bit offsets;
+// The LDS tiles, and the 128-token copy tile for INT4 with a K past the wide tile's 32-bit offsets;
 // returns the K split whose partials it left in ws (1: y holds the product).
 template <int FMT>
 int launch_tiles(const void* x, const void* qw, const void* sc, const void* zp, void* y, int M, int K, int N,
@@ -1181,7 +1181,7 @@ long long gemm_workspace_bytes(int M, int K, int N) {
     for (const Plan& p : {plan_gemm(M, K, N, true), plan_gemm(M, K, N, false), plan_lds(M, K, N)})
         if (p.split > 1) bytes = std::max(bytes, (long long)p.split * M * N * 4);
     for (int fmt : {(int)kInt4G32, (int)kFp8E4M3})
-        if (wide_any_shape(fmt, K, N)) {
+        if (wide_any_shape(K)) {
             const int split = wide_choice(fmt, M, K, N).split;
             if (split > 1) bytes = std::max(bytes, (long long)split * M * N * 4);
         }
@@ -1222,7 +1222,7 @@ MOSS_API int moss_w4g32_gemm_silu(const void* x, const void* qw, const void* sc,
     MOSS_CHECK_ARG(MOSS_ALIGNED(x, 16) && MOSS_ALIGNED(qw, 16) && workspace_bytes >= 0);
     hipStream_t st = (hipStream_t)stream;
     if (silu_fusable_shape(M, K, N) && MOSS_ALIGNED(y, 8) && MOSS_ALIGNED(sc, 16) && MOSS_ALIGNED(zp, 8)) {
-        if (wide_shape(kInt4G32, K, 2 * N))
+        if (wide_silu_shape(K, N))
             return wide_launch_w4(kWideSilu, wide_plan(kInt4G32, M, K, 2 * N, 1, 1),
                                   WideArgs{x, qw, sc, zp, nullptr, y, nullptr, M, K, N, QkRope{}}, st);
         const dim3 grid((unsigned)(((M + 127) / 128) * ((N + 63) / 64)));
@@ -1235,7 +1235,7 @@ MOSS_API int moss_w4g32_gemm_silu(const void* x, const void* qw, const void* sc,
     MOSS_CHECK_ARG(workspace && MOSS_ALIGNED(workspace, 16) && workspace_bytes >= inter);
     char* ws = (char*)workspace;
     WidePlan wp;
-    if (!tokens_gemv(M, K, x, qw) && MOSS_ALIGNED(y, 8) &&
+    if (!tokens_gemv(M, K, x, qw) && MOSS_ALIGNED(y, 8) && wide_silu_shape(K, N) &&
         choose_wide(kInt4G32, M, K, 2 * N, x, qw, sc, zp, ws, ws + inter, workspace_bytes - inter, wp) && wp.split == 1 && !wp.any)
         return wide_launch_w4(kWideSilu, wp, WideArgs{x, qw, sc, zp, nullptr, y, nullptr, M, K, N, QkRope{}}, st);
     int split = 1;

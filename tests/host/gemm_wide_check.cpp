@@ -31,11 +31,14 @@ struct Watched {
     }
 };
 
-static std::vector<char> operand(size_t bytes) {
-    std::vector<char> v(std::max<size_t>(bytes, 1));
-    operands.push_back({v.data(), bytes});
-    return v;
-}
+// Never touched, so a large one costs no memory.
+struct Untouched {
+    char* p;
+    explicit Untouched(size_t bytes) : p((char*)malloc(std::max<size_t>(bytes, 1))) { operands.push_back({p, bytes}); }
+    ~Untouched() { free(p); }
+    Untouched(const Untouched&) = delete;
+    const char* data() const { return p; }
+};
 
 static int runs;
 static bool check(int fmt, int r, int jt, int split, bool any, WideEpilogue epi, int M, int N, int K) {
@@ -43,8 +46,8 @@ static bool check(int fmt, int r, int jt, int split, bool any, WideEpilogue epi,
     const int nw = epi == kWideSilu ? 2 * N : N, G = K / 32, L = 64, before = (int)violations;
     const bool int4 = fmt == kInt4G32;
     operands.clear();
-    std::vector<char> x = operand((size_t)M * K * 2), qw = operand((size_t)nw * K / (int4 ? 2 : 1)),
-                      sc = operand(int4 ? (size_t)nw * G * 2 : 0), zp = operand(int4 ? (size_t)nw * G / 2 : 0);
+    const Untouched x((size_t)M * K * 2), qw((size_t)nw * K / (int4 ? 2 : 1)), sc(int4 ? (size_t)nw * G * 2 : 0),
+        zp(int4 ? (size_t)nw * G / 2 : 0);
     Watched<uint16_t> y((size_t)M * (epi == kWideQkRope ? 4096 : N)), kc(8 * L * 128), vc(8 * L * 128);
     Watched<float> part(epi == kWideSplit ? (size_t)p.split * M * N : 1);
     std::vector<float> scale(int4 ? 1 : N);
@@ -83,6 +86,14 @@ static bool bounds() {
                     // shares of K past its end among them
                     for (int split : {2, 4}) ok &= check(fmt, r, jt, split, true, kWideSplit, 33, n, k);
                 }
+        }
+    // weights past 4 GiB: the last workgroups' rows
+    last_blocks = 3;
+    for (int fmt : {(int)kInt4G32, (int)kFp8E4M3})
+        for (int r : {1, 2}) {
+            const int n = (1 << (fmt == kInt4G32 ? 21 : 20)) + 132;
+            ok &= check(fmt, r, 4, 1, false, kWidePlain, 3, n, 4096);
+            ok &= check(fmt, r, 4, 2, true, kWideSplit, 3, n + 1, 4096);
         }
     printf("%d launches\n", runs);
     return ok;

@@ -124,6 +124,7 @@ C __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, A, C c, int, int, int) { return c; 
 
 // -------------------------------------------------------------- a launch
 inline bool run_launches = true;
+inline unsigned last_blocks = ~0u;  // run only this many
 struct Launched {
     const char* kernel;
     unsigned blocks;
@@ -136,7 +137,7 @@ void host_launch(const char* kernel, dim3 grid, dim3 block, F lane) {
     gridDim = grid;
     blockDim = block;
     for (blockIdx.y = 0; blockIdx.y < grid.y; ++blockIdx.y)
-        for (blockIdx.x = 0; blockIdx.x < grid.x; ++blockIdx.x)
+        for (blockIdx.x = grid.x > last_blocks ? grid.x - last_blocks : 0; blockIdx.x < grid.x; ++blockIdx.x)
             for (threadIdx.x = 0; threadIdx.x < block.x; ++threadIdx.x) lane();
 }
 #define hipLaunchKernelGGL(kernel, grid, block, lds, stream, ...) \

@@ -81,3 +81,23 @@ def test_qk_rope_equals_gemm_then_qk_rope(dev, m):
     q2 = pointwise.qk_rope(w4g32.gemm(x, w), qn, kn, cos, sin, k2, v2, pos, 1e-6, cos_by_position=True)
     for a, b in ((q1.contiguous(), q2.contiguous()), (k1, k2), (v1, v2)):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("m", [5, 40, 130])
+def test_weight_past_2_gib(dev, m):
+    """Rows at both ends of a weight whose codes pass 2 GiB, against the same rows as weights of their own: one
+    sum order, so bit for bit (32772 rows fill the card as the whole does, so neither splits K)."""
+    from moss_tts._runtime import w4g32
+
+    k, n = 1024, 2 ** 22 + 132
+    print(f"wide large weight M={m}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(m)
+    qw = torch.randint(-2 ** 31, 2 ** 31 - 1, (n, k // 8), device=dev, generator=g, dtype=torch.int32)
+    scales = (0.01 + 0.01 * torch.rand((n, k // 32), device=dev, generator=g)).bfloat16()
+    zeros = torch.randint(0, 256, (n, k // 64), device=dev, generator=g, dtype=torch.uint8)
+    assert qw.numel() * 4 > 2 ** 31
+    x = torch.randn((m, k), device=dev, generator=g).bfloat16()
+    y = w4g32.gemm(x, w4g32.PackedW4G32(qw, scales, zeros))
+    for lo in (0, n - 32772):
+        part = w4g32.PackedW4G32(qw[lo:lo + 32772], scales[lo:lo + 32772], zeros[lo:lo + 32772])
+        assert torch.equal(y[:, lo:lo + 32772], w4g32.gemm(x, part))
