@@ -1,6 +1,8 @@
 // Host checks of the wide GEMM tile, compiled against hip_on_host.h.
 //   bounds          every instance, over remainders of M, N and K: addresses of every read, and stores
-//   plan            reads "format M K N" lines, prints what the dispatch picks for each
+//   plan            reads "format M K N" lines (0 INT4, 1 e4m3, 2 INT4 gate||up + SiLU of N outputs, 3 INT4 q||k||v +
+//                   RoPE), prints what the dispatch picks for each: r, jt, split, any, workspace
+//                   (the LDS tiles: -rows, columns, split; neither: 0)
 #include "w4g32_gemm.hip"
 
 namespace moss {
@@ -106,9 +108,22 @@ int main(int argc, char** argv) {
     const void* p = (const void*)4096;  // aligned for everything, never read
     while (scanf("%d %d %d %d", &fmt, &M, &K, &N) == 4) {
         WidePlan w{};
-        const long long ws = gemm_workspace_bytes(M, K, N);
-        if (!(fmt == kInt4G32 && tokens_gemv(M, K, p, p))) {
-            if (!choose_wide(fmt, M, K, N, p, p, p, p, p, p, ws, w)) w = WidePlan{};
+        const long long ws = gemm_workspace_bytes(M, K, fmt == 2 ? 2 * N : N);
+        if (fmt == 2) {  // gate||up with the SiLU epilogue, N outputs
+            const bool fused = silu_fusable_shape(M, K, N);
+            if (fused && wide_silu_shape(K, N)) w = wide_plan(kInt4G32, M, K, 2 * N, 1, 1);
+            else if (fused || tokens_gemv(M, K, p, p) || !wide_silu_shape(K, N) ||
+                     !choose_wide(kInt4G32, M, K, 2 * N, p, p, p, p, p, p, ws, w) || w.split > 1 || w.any) w = WidePlan{};
+        } else if (fmt == 3) {  // q||k||v with the q/k norm + RoPE epilogue
+            if (qk_rope_fusable_shape(M, K) && wide_shape(kInt4G32, K, kQkvN)) w = wide_plan(kInt4G32, M, K, kQkvN, 1, 1);
+        } else if (!(fmt == kInt4G32 && tokens_gemv(M, K, p, p))) {
+            if (!choose_wide(fmt, M, K, N, p, p, p, p, p, p, ws, w)) {
+                w = WidePlan{};
+                if (!stream_shape(fmt, M, K, N, p, p, p, p, p)) {
+                    const Plan t = plan_gemm(M, K, N, fmt == kInt4G32);
+                    w = WidePlan{t.reg ? 0 : -t.bm, t.bn, t.split, false, 0};
+                }
+            }
         }
         printf("%d %d %d %d %lld\n", w.r, w.jt, w.split, (int)w.any, ws);
     }

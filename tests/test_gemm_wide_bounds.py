@@ -8,6 +8,7 @@ import subprocess
 
 import pytest
 
+import test_gpu_gemm_wide
 from moss_tts import _build
 
 HOST = os.path.join(os.path.dirname(os.path.abspath(__file__)), "host")
@@ -43,8 +44,8 @@ def test_reads_and_stores_stay_in_bounds(gemm_wide_check):
 
 
 def _plans(check, calls):
-    """(r, jt, split, any, workspace bytes) of each (format, M, K, N) call with aligned operands; r = 0: not the
-    wide tile."""
+    """(r, jt, split, any, workspace bytes) of each (format, M, K, N) call with aligned operands in the wide tile,
+    (-rows, columns, split, 0, bytes) in the LDS tiles, zeros elsewhere."""
     text = "\n".join(" ".join(map(str, c)) for c in calls)
     r = subprocess.run([check, "plan"], input=text, capture_output=True, text=True, check=True)
     return [tuple(map(int, line.split())) for line in r.stdout.splitlines()]
@@ -56,7 +57,7 @@ def test_offsets_fit_32_bits(gemm_wide_check):
     calls = [(f, 160, k, 4) for f in (0, 1) for k in (last, last + 256, 2 ** 24)]
     assert [p[0] > 0 for p in _plans(gemm_wide_check, calls)] == [True, False, False] * 2
     large = [(0, 33, 4096, 2 ** 20 + 4), (0, 160, 4096, 2 ** 21), (1, 160, 4096, 2 ** 20 + 4)]
-    assert all(p[0] for p in _plans(gemm_wide_check, large))
+    assert all(p[0] > 0 for p in _plans(gemm_wide_check, large))
 
 
 def _earlier_split(m, k, n):
@@ -83,5 +84,25 @@ def test_slower_calls_stay_out_of_the_wide_tile(gemm_wide_check):
               (0, 6, 12288, 4096), (1, 6, 12288, 4096), (1, 7, 4096, 12288), (1, 8, 4096, 6144)]
     faster = [(0, 424, 4160, 1701), (0, 150, 4160, 1001), (0, 10, 4160, 1506), (0, 154, 6976, 83), (1, 53, 6400, 3434),
               (1, 582, 4352, 102), (1, 64, 4096, 12288), (0, 24, 12288, 4096), (1, 16, 12288, 4096), (1, 17, 4096, 6144)]
-    assert not any(p[0] for p in _plans(gemm_wide_check, slower))
-    assert all(p[0] for p in _plans(gemm_wide_check, faster))
+    assert all(p[0] <= 0 for p in _plans(gemm_wide_check, slower))
+    assert all(p[0] > 0 for p in _plans(gemm_wide_check, faster))
+
+
+def test_every_instance_has_its_gpu_case(gemm_wide_check):
+    """The GPU cases run the instances that they name, and they name every compiled one but the regular splits of
+    256 rows by 96 (INT4) and 128 tokens, which the dispatch picked for none of 400000 calls of up to 2900 tokens, K =
+    16384 and N = 32768."""
+    cases = test_gpu_gemm_wide.INSTANCES
+    plans = _plans(gemm_wide_check, [(i[0], *c) for i, c in cases.items()])
+    assert [(i[0], r, jt, any_, int(split > 1)) for i, (r, jt, split, any_, _) in zip(cases, plans)] == list(cases)
+    tiles = [(1, jt) for jt in range(1, 6)] + [(2, 3), (2, 4)]
+    regular = {(f, *t, 0, s) for f in (0, 1) for t in tiles for s in (0, 1)} | {(1, 2, 5, 0, s) for s in (0, 1)}
+    any_shape = {(f, *t, 1, s) for f in (0, 1) for t in tiles if t not in ((1, 3), (2, 3)) for s in (0, 1)}
+    fused = {(f, *t, 0, 0) for f in (2, 3) for t in tiles}
+    assert set(cases) == regular - {(0, 2, 3, 0, 1), (0, 2, 4, 0, 1), (1, 2, 4, 0, 1)} | any_shape | fused
+
+
+def test_gpu_cases_of_the_lds_tiles(gemm_wide_check):
+    cases = test_gpu_gemm_wide.TILES_IN_LDS
+    plans = _plans(gemm_wide_check, [(i[0], *c) for i, c in cases.items()])
+    assert [(i[0], -r, bn, split) for i, (r, bn, split, *_) in zip(cases, plans)] == [i[:4] for i in cases]

@@ -291,11 +291,11 @@ def test_gemv_tokens_equal_single_token_gemv(dev, k, n):
                                    (37, 4096, 32800), (512, 4096, 6144), (512, 12288, 4096), (512, 4096, 4096),
                                    # the 128 x 128 tile at full size, with ragged M and N, and an odd step count
                                    (512, 4096, 24576), (300, 1024, 32808), (260, 1088, 16448),
-                                   # register-weight tile with a 16-group last zero-point chunk (G = 144)
+                                   # a 16-group last zero-point chunk (G = 144)
                                    (260, 4608, 12296),
-                                   # 32- and 64-token register tiles with a K split, ragged N
+                                   # few tokens with a K split, ragged N
                                    (5, 1024, 1000), (16, 4096, 4096), (48, 4608, 2056),
-                                   # N % 4 != 0: the LDS tiles take shapes the register tile would
+                                   # N % 4 != 0: no quads of outputs
                                    (40, 4096, 1001), (130, 4096, 258),
                                    # the small-M weight-streaming kernel (M <= 32, K % 4096 == 0): one
                                    # and two token tiles, ragged tiles, a ragged last row tile, K = 12288
@@ -416,8 +416,8 @@ def test_gemm_add_rmsnorm_equals_gemm_then_add_rmsnorm(dev, m, k, n):
 @pytest.mark.parametrize("m,k,n", [(512, 4096, 4096), (48, 4096, 2056)])
 def test_gemm_fallbacks_match(dev, m, k, n):
     """The C-ABI's fallbacks give the same products: without a workspace the planned K split is
-    dropped (one pass over K), and scales or zero points that are not 16 / 8-byte aligned send the
-    register-weight tile's shapes to the LDS tiles.  Against the oracle at the GEMM tolerance."""
+    dropped (one pass over K), and scales or zero points that are not 16 / 8-byte aligned leave the wide
+    tile's regular form for its any-shape form or the LDS tiles.  Against the oracle at the GEMM tolerance."""
     from moss_tts._runtime import native
 
     print(f"gemm fallbacks M={m} K={k} N={n}", flush=True)
