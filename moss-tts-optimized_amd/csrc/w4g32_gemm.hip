@@ -1059,27 +1059,29 @@ bool split_fits(int split, const void* ws, long long ws_bytes, const void* y, in
 }
 
 // Where the weight-streaming kernel, which never splits K over workgroups, still beats the wide tile with
-// its partial sums: few activations to read in each workgroup (M K), by the format and for up to one workgroup
-// per CU (N <= 4096) or more.  Streamed / wide, us, weights from memory:
+// its partial sums: few activations to read in each workgroup (M K), for up to one workgroup per CU (N <=
+// 4096) or, e4m3, more.  Streamed / wide, us, weights from memory:
 //   INT4 N = 4096: K = 4096 M = 16 7.8 / 8.9, 21 9.6 / 9.4, 24 10.2 / 9.6; K = 12288 M = 6 14.3 / 15.7, 7 15.1 / 15.8,
 //        8 15.6 / 15.8, 12 17.3 / 16.0;  N = 6144: M = 5 10.6 / 10.2, 8 11.8 / 10.4
 //   e4m3 N = 4096, K = 12288: M = 6 14.4 / 17.6, 12 17.4 / 17.8, 14 18.2 / 17.7;  N = 6144: M = 6 10.6 / 11.7, 12 12.3 / 12.1;
-//        N = 12288: M = 6 16.0 / 18.7, 12 17.7 / 19.1, 15 18.8 / 19.1;  N = 24576: M = 12 32.7 / 32.7, 14 33.7 / 32.4
+//        N = 12288: M = 6 16.0 / 18.7, 8 16.8 / 18.8, 15 18.8 / 19.1;  N = 24576: M = 12 32.7 / 32.7, 14 33.7 / 32.4
+// With weights partly in the last-level cache, where a repeated call finds them, the e4m3 bounds lie lower (N =
+// 12288: M = 8 16.4 / 14.8; K = 12288: M = 6 13.4 / 14.9, 8 15.5 / 13.9): they are set between the two.
 bool stream_better(int fmt, int M, int K, int N) {
     const long long mk = (long long)M * K;
-    if (N <= 4096) return mk <= (fmt == kInt4G32 ? 21 : 38) * 4096;
-    return fmt == kFp8E4M3 && mk <= 13 * 4096;
+    if (N <= 4096) return mk <= 21 * 4096;
+    return fmt == kFp8E4M3 && mk <= (N >= 16384 ? 12 : 5) * 4096;
 }
 
 // Whether the wide tile (gemm_wide_kernel.h) takes a call, and how.  Shapes without whole blocks of K or
 // quads of N and misaligned pointers take its any-shape form, e4m3 the regular one too, where it is expected to
 // take less time than the LDS tiles.  A short K, whose steps the any-shape form rounds up to a block of four, and
 // 33 to 64 tokens over many rows stay in those (M = 424, K = 832, N = 11701: 22.4 us there, 34.6 in the wide
-// tile; e4m3 M = 53, K = 1536, N = 13434: 11.6, 16.5).  40000 random calls (INT4 and e4m3, M = 2 .. 1024, K = 256 ..
-// 12288, N = 64 .. 16384) take 0.67 of the time they took in the LDS tiles and the streaming kernel in the mean, and
-// 0.2% of them over 1.05 times; with the wide tile wherever it can run 7% did.  A plan whose partial sums do not
-// fit the workspace is split less, or left to the streaming kernel where that takes the shape (K = N = 4096, M =
-// 24: 10 us against 24 us unsplit).
+// tile; e4m3 M = 53, K = 1536, N = 13434: 11.6, 16.5).  17000 random calls (INT4 and e4m3, M = 2 .. 1024, K = 256 ..
+// 12288, N = 64 .. 16384, weights from memory) take 0.64 of the time they took in the LDS tiles and the streaming
+// kernel in the mean, and 0.9% of them over 1.05 times (0.3% without the few e4m3 tokens above); with the wide tile
+// wherever it can run 7% did.  A plan whose partial sums do not fit the workspace is split less, or left to the
+// streaming kernel where that takes the shape (K = N = 4096, M = 24: 10 us against 24 us unsplit).
 bool choose_wide(int fmt, int M, int K, int N, const void* x, const void* qw, const void* sc, const void* zp,
                  const void* y, const void* ws, long long ws_bytes, WidePlan& p) {
     const bool aligned = MOSS_ALIGNED(y, 8) && (fmt == kFp8E4M3 || (MOSS_ALIGNED(sc, 16) && MOSS_ALIGNED(zp, 8)));

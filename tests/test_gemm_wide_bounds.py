@@ -81,7 +81,7 @@ def test_slower_calls_stay_out_of_the_wide_tile(gemm_wide_check):
     neighbours of theirs that take 0.2 to 0.9 of the time in it."""
     slower = [(0, 424, 832, 11701), (0, 595, 320, 12317), (0, 1003, 320, 5991), (0, 10, 576, 1506), (0, 47, 1088, 6207),
               (0, 12, 320, 13373), (1, 53, 1536, 13434), (1, 62, 1600, 9892), (1, 60, 4096, 4096),
-              (0, 6, 12288, 4096), (1, 6, 12288, 4096), (1, 7, 4096, 12288), (1, 8, 4096, 6144)]
+              (0, 6, 12288, 4096), (1, 6, 12288, 4096)]
     faster = [(0, 424, 4160, 1701), (0, 150, 4160, 1001), (0, 10, 4160, 1506), (0, 154, 6976, 83), (1, 53, 6400, 3434),
               (1, 582, 4352, 102), (1, 64, 4096, 12288), (0, 24, 12288, 4096), (1, 16, 12288, 4096), (1, 17, 4096, 6144)]
     assert all(p[0] <= 0 for p in _plans(gemm_wide_check, slower))
