@@ -414,7 +414,9 @@ MOSS_API int moss_embedding_sum(const void* ids, const void* text, const void* a
     MOSS_CHECK_ARG(ids && text && audio && out && T > 0 && H > 0 && Vt > 0 && V > 0 && Q >= 0);
     // 16- or 8-byte loads where rows allow them: 512 tokens x 33 rows of 4096 in 50 us with 2-byte loads
     // -- and one value per thread for a few tokens, whose time is the chain of 33 rounded additions per value
-    // and not the loads (one token: the decode step 237.5 -> 235.7 us, its W4A8 form 221.8 -> 219.0)
+    // and not the loads (1 / 2 / 4 tokens of 4096 with eight values per thread: 7.3 / 7.4 / 7.9 us, with one 4.8 / 4.9 /
+    // 5.1; 2 of 8192 7.8 / 5.2; past 4 x 4096 values not measured.  A decode step of four layers differs by less than
+    // two runs of it do)
     const bool few = (long long)T * H <= 4 * 4096;
     if (!few && H % 8 == 0 && MOSS_ALIGNED(text, 16) && MOSS_ALIGNED(audio, 16) && MOSS_ALIGNED(out, 16))
         hipLaunchKernelGGL(embedding_sum_rows<8>, dim3(T, (H / 8 + 255) / 256), dim3(256), 0, (hipStream_t)stream,

@@ -1,4 +1,4 @@
-// The prompt GEMM tile whose waves own 32 or 64 weight rows over 32 JT tokens (gemm_wide.hip).
+// The prompt GEMM tile whose waves own 32 or 64 weight rows over 32 JT tokens (gemm_wide_kernel.h).
 #pragma once
 
 #include "common.h"

@@ -12,7 +12,8 @@ namespace {
 // fewer busy CUs hold a higher clock and a step takes down to 0.75 of this.  By these costs the chosen
 // tile and split, with the partial sums' cost, was the best measured one at 34 of the 45 shapes, within 6%
 // of it at 41 and within 17% at all.  0: no such instance (R = 2 below 3 token tiles was nowhere the best,
-// and INT4 at 2 x 5 spills).
+// and INT4 at 2 x 5, with scales and zero points besides, spills in the loop; e4m3 there spills two registers and is
+// the fastest tile all the same: M = 777, N = 12288 72 us).
 struct StepCost {
     int alone[5], shared[5];
 };
@@ -54,11 +55,10 @@ int launch_tile(WideEpilogue epi, const WidePlan& p, const WideArgs& a, hipStrea
 bool wide_any_shape(int K) { return K % kStep == 0 && 320ll * K < 1ll << 32; }
 
 // Whole blocks of four K steps and 4-output stores; INT4: the 8 zero bytes of every block on one
-// nibble side of their 128-group chunk (the last chunk a multiple of 16 groups long).
+// nibble side of their 128-group chunk (the last chunk a multiple of 16 groups long, as K / 32 is then).
 bool wide_shape(int fmt, int K, int nw) {
     if (nw % 4 || K % (4 * kStep) || !wide_any_shape(K)) return false;
-    const int G = K / 32;
-    return fmt == kFp8E4M3 || (G % 16 == 0 && (G % 128) % 16 == 0);
+    return fmt == kFp8E4M3 || K / 32 % 16 == 0;
 }
 
 // A SiLU workgroup reaches from its gate rows to the up rows, N of K / 2 bytes further on.

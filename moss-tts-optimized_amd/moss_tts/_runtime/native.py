@@ -133,7 +133,8 @@ def workspace(nbytes: int, device) -> tuple:
 
 
 # Plain integers: ctypes converts them by the declared argument types, and a c_void_p object per pointer
-# and a torch Stream object per call took 4 us of the 22 us of a one-token projection.
+# and a torch Stream object per call took 4 us of the 22 us of a one-token projection.  The stream's handle comes
+# from a private name of torch (2.10 has it; torch.cuda.current_stream(t.device).cuda_stream is the public way).
 def stream_of(t: torch.Tensor) -> int:
     return torch._C._cuda_getCurrentRawStream(t.get_device())
 
