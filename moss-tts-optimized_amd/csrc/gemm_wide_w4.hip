@@ -12,8 +12,7 @@ namespace {
 // fewer busy CUs hold a higher clock and a step takes down to 0.75 of this.  By these costs the chosen
 // tile and split, with the partial sums' cost, was the best measured one at 34 of the 45 shapes, within 6%
 // of it at 41 and within 17% at all.  0: no such instance (R = 2 below 3 token tiles was nowhere the best,
-// and INT4 at 2 x 5, with scales and zero points besides, spills in the loop; e4m3 there spills two registers and is
-// the fastest tile all the same: M = 777, N = 12288 72 us).
+// and INT4 at 2 x 5 spills; e4m3 at 2 x 5 keeps two registers in scratch, outside its loop).
 struct StepCost {
     int alone[5], shared[5];
 };
