@@ -175,7 +175,7 @@ def quantize_launch(w: torch.Tensor, symmetric: bool):
     _require(_aligned(w, 16), "w must be 16-byte aligned")
     n, k = w.shape
     out = PackedW4G32.empty(n, k, w.device)
-    bad = torch.empty(1, dtype=torch.int32, pin_memory=True)
+    bad = torch.empty(1, dtype=torch.int32, device="cpu", pin_memory=True)
     bad[0] = 0
     stream = torch.cuda.current_stream(w.device)
     native.call("moss_w4g32_quantize_checked", native.ptr(w), native.ptr(out.qw), native.ptr(out.scales),

@@ -34,3 +34,15 @@ def test_scale_range(dev, symmetric, n, k, group):
         scales = quantize(w).scales.view(-1)
         others = torch.arange(scales.numel(), device=dev) != group
         assert scales.isfinite().all() and torch.equal(scales[others], plain.scales.view(-1)[others])
+
+
+@pytest.mark.parametrize("symmetric", [False, True])
+def test_under_a_default_device(dev, symmetric):
+    """A module made where a program has set the device for its new tensors."""
+    from moss_tts._runtime.modules import QuantLinearG32
+
+    w = torch.randn((8, 64), device=dev)
+    with torch.device(dev):
+        inside = QuantLinearG32.from_float(w, symmetric=symmetric)
+    outside = QuantLinearG32.from_float(w, symmetric=symmetric)
+    assert torch.equal(inside.qw, outside.qw) and torch.equal(inside.scales, outside.scales)
