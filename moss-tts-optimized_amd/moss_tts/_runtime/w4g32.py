@@ -179,7 +179,7 @@ def quantize_launch(w: torch.Tensor, symmetric: bool):
     bad[0] = 0
     stream = torch.cuda.current_stream(w.device)
     native.call("moss_w4g32_quantize_checked", native.ptr(w), native.ptr(out.qw), native.ptr(out.scales),
-                native.ptr(out.zeros), native.ptr(bad), k, n, int(symmetric), stream.cuda_stream)
+                native.ptr(out.zeros), native.ptr(bad), k, n, int(bool(symmetric)), stream.cuda_stream)
 
     def check() -> None:
         stream.synchronize()
