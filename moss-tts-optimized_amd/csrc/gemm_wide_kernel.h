@@ -410,9 +410,10 @@ __global__ __launch_bounds__(256, 2) void gemm_wide_kernel(
     // l % 32; the four e of a quad are consecutive n
     if constexpr (ANY) {
         if (N % 4 || (EPI == kWidePlain && reinterpret_cast<uintptr_t>(Y) % 8)) {
-            // No quads: a store of one value per lane would touch a row per lane, so each 128-row half of the tile goes through the LDS of the ring, fp32 by token row
-            // (row t in buffer (t / 8) % 4, 16-byte chunk c at c ^ (t & 31)), and leaves row by row
-            // (M = 595, K = 320, N = 12317: 32.2 -> 21.4 us; M = 150, K = 4160, N = 1001: 17.0 -> 14.0).
+            // No quads: a store of one value per lane would touch a row per lane, so each 128-row half of the tile
+            // goes through the LDS of the ring, fp32 by token row (row t in buffer (t / 8) % 4, 16-byte chunk c at
+            // c ^ (t & 31)), and leaves row by row (M = 595, K = 320, N = 12317: 32.2 -> 21.4 us; M = 150, K = 4160,
+            // N = 1001: 17.0 -> 14.0).
             auto chunk = [&](int row, int c) {
                 const int b = (row >> 3) & 3;
                 uint16_t* x = b == 0 ? X0 : b == 1 ? X1 : b == 2 ? X2 : X3;
